@@ -6,7 +6,7 @@
 // arcsin/arccos; here the same quantities come from the vector components
 // (sin lat = y/|v|, cos lat = sqrt(x^2+z^2)/|v|, cos lng = z/sqrt(x^2+z^2), ...),
 // which is the same arithmetic up to rounding, with no transcendental calls in
-// the loop.  Quirks kept: the latitude-0 substitution lat = 1e-6 rad
+// the loop, and a path after its one refraction is followed as a straight line.  Quirks kept: the latitude-0 substitution lat = 1e-6 rad
 // (shape.py:231-233), the next-shell radius taken at the current point's
 // latitude (raypath.py:182), refraction only at the first boundary
 // (raypath.py:158, 257), the numpy arange trial grid and linear root of
@@ -81,25 +81,35 @@ __device__ inline Surf ellipse(const Geo &G, double a, const LatLng &q) {
     return s;
 }
 
-// the shell quantities at a path point v that depend only on its latitude: f, the radius of
-// the unit-equatorial-radius ellipse there (a shell of equatorial radius a has a f), and the
-// shell normal n.  With X = x^2 + z^2, Y = y^2 and sin lat = y/|v|, cos lat = sqrt(X)/|v|,
-// ellipse() reduces to f = sqrt((X + ratio^2 Y) / (X + Y)) and
-// n = (ratio x, y, ratio z) rsqrt(ratio^2 X + Y) (the same values up to rounding, with one
-// division, one square root and one reciprocal square root in parallel instead of latlng's and
-// ellipse's chain: ray paths 0.66 -> 0.41 ms on 16384 rays of 800 layers).  y == 0 takes the
-// 1e-6 rad latitude substitution through latlng.
-__device__ inline void shell_at(const Geo &G, V3 v, double &f, V3 &n) {
-    if (v.y == 0.0) {
-        const Surf s = ellipse(G, 1.0, latlng(v));
-        f = s.rmag;
-        n = s.n;
-        return;
-    }
-    const double X = v.x * v.x + v.z * v.z, Y = v.y * v.y, r2 = G.ratio * G.ratio;
-    f = sqrt(fma(r2, Y, X) / (X + Y));
-    const double inv = rsqrt(fma(r2, X, Y));
-    n = {G.ratio * v.x * inv, v.y * inv, G.ratio * v.z * inv};
+// sqrt of a finite x >= 0 (NaN below 0, as sqrt): the hardware reciprocal square root refined
+// by one coupled Newton step and one correction of the root, without the range scaling of the
+// library's (arguments here are squared km, far from FP64's limits): about an ulp in 8
+// dependent operations.
+__device__ inline double sqrt_km2(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double e = fma(-h, g, 0.5);
+    g = fma(g, e, g);
+    h = fma(h, e, h);
+    g = fma(fma(-g, g, x), h, g);
+    return __builtin_amdgcn_class(x, 0x260) ? x : g;   // +-0 and +inf are their own roots
+}
+
+// 1 / x for a positive finite x: the hardware estimate refined twice
+__device__ inline double rcp_pos(double x) {
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(r, fma(-x, r, 1.0), r);
+    return fma(r, fma(-x, r, 1.0), r);
+}
+
+// f^2 of the shells at a point: a shell of equatorial radius a has radius a f at the point's
+// latitude, f^2 = (X + ratio^2 Y) / (X + Y) = 1 - (1 - ratio^2) y^2 / |v|^2 with X = x^2 + z^2 and
+// Y = y^2 (ellipse() with sin lat = y / |v|, cos lat = sqrt(X) / |v|).  y == 0 takes the
+// reference's 1e-6 rad latitude (kLat0 = sin^2 of it).
+constexpr double kLat0 = 9.999999999998333e-07 * 9.999999999998333e-07;
+__device__ inline double shell_f2(double flat, double y, double q) {
+    const double s2 = y == 0.0 ? kLat0 : y * y * rcp_pos(q);
+    return fma(-flat, s2, 1.0);
 }
 
 // Rays per block.  One thread per ray: a ray's path is one dependent chain of FP64 steps, so
@@ -107,8 +117,10 @@ __device__ inline void shell_at(const Geo &G, V3 v, double &f, V3 &n) {
 // line sums (rbx_alpha) when a caller puts it on a second stream or graph branch; four
 // wavefronts per block keep it on a quarter as many CUs as one per block, leaving the other
 // CUs' slots whole for the line sums: 800 layers x 1024 frequencies x 16384 rays, graph step
-// 3.71 -> 3.47 ms (the paths alone 0.42 -> 0.45 ms; 2 and 8 wavefronts per block: 3.59, 3.53 ms).
+// 3.71 -> 3.47 ms when the paths alone took 0.42 -> 0.45 ms (2 and 8 wavefronts per block: 3.59,
+// 3.53 ms).
 constexpr int kRayThreads = 256;
+constexpr int kWin = 8;   // shell radii fetched per window
 
 struct RayArgs {
     Geo G;
@@ -127,6 +139,8 @@ struct RayArgs {
     int natm;
 };
 
+// SEC: limb 'sec' (raypath.py:218-219)
+template <bool SEC>
 __global__ __launch_bounds__(kRayThreads) void raypath_kernel(RayArgs A) {
     const int ray = blockIdx.x * blockDim.x + threadIdx.x;
     if (ray >= A.nray) return;
@@ -156,31 +170,34 @@ __global__ __launch_bounds__(kRayThreads) void raypath_kernel(RayArgs A) {
     const double mu = sqrt(1.0 - tmp);
 
     // ---- findEdge: trial zQ = arange(1.01 sqrt(1-b^2), 0, -0.005) ----
-    const double start = sqrt(1.0 - tmp) * 1.01;
+    // a trial lies below the top shell when |v| < f, that is |v|^2 < f^2: no root per trial;
+    // the distances of the two bracketing trials are formed once the bracket is known
+    const double start = mu * 1.01;
     const int ntrial = static_cast<int>(ceil((0.0 - start) / -0.005));
     const double z1 = start + -0.005;
     const double dz = z1 - start;
-    double zprev = 0.0, dprev = 0.0, zhit = 0.0, dhit = 0.0;
+    const double flat = 1.0 - G.ratio * G.ratio;
+    auto trial = [&](int i) { return (i == 0) ? start : ((i == 1) ? z1 : start + i * dz); };
     int hit = -1;
     for (int i = 0; i < ntrial; ++i) {
-        const double zq = (i == 0) ? start : ((i == 1) ? z1 : start + i * dz);
-        const V3 bv = mat(G.M, V3{b0, b1, zq});
-        const double r1 = norm(bv) * rNorm;
-        const Surf s = ellipse(G, rNorm, latlng(bv));
-        const double dd = r1 - s.rmag;
-        if (r1 < s.rmag) {
+        const V3 bv = mat(G.M, V3{b0, b1, trial(i)});
+        const double q = dot(bv, bv), Y = bv.y * bv.y;
+        // q < f^2 times q > 0 (1e-6 rad at y == 0)
+        if (q * q < fma(-flat, bv.y == 0.0 ? kLat0 * q : Y, q)) {
             hit = i;
-            zhit = zq;
-            dhit = dd;
             break;
         }
-        zprev = zq;
-        dprev = dd;
     }
     if (hit < 0) {
         A.nsteps[ray] = -1;
         return;
     }
+    auto above = [&](double z) {   // |v| - top shell radius at v's latitude
+        const V3 bv = mat(G.M, V3{b0, b1, z});
+        return norm(bv) * rNorm - ellipse(G, rNorm, latlng(bv)).rmag;
+    };
+    const double zhit = trial(hit), dhit = above(zhit);
+    const double zprev = hit > 0 ? trial(hit - 1) : 0.0, dprev = hit > 0 ? above(zprev) : 0.0;
     // np.interp(0, [dhit, dprev], [zhit, zprev]) on the two bracketing trials
     double zq;
     if (hit == 0 || dhit == 0.0) {
@@ -193,46 +210,74 @@ __global__ __launch_bounds__(kRayThreads) void raypath_kernel(RayArgs A) {
     const V3 edge = rNorm * mat(G.M, V3{b0, b1, zq});
 
     // ---- compute_ds: start on the top shell at the edge's latitude ----
-    const LatLng q = latlng(edge);
-    const Surf geo = ellipse(G, rNorm, q);
+    const LatLng q0 = latlng(edge);
+    const Surf geo = ellipse(G, rNorm, q0);
     V3 s = mat(G.M, V3{0.0, 0.0, -1.0});
     V3 r = geo.r;
-    V3 n = geo.n;
-    double c = -dot(s, n);                            // cos(t_inc)
-    double nratio = Nl[0] / Nl[1];
-    double st = nratio * sqrt(1.0 - c * c);          // sin(t_tran)
-    double ct = sqrt(1.0 - st * st);                 // cos(t_tran)
-    const double cm_half = (A.units == 1);
-    int layer = 0;
+    {
+        // refraction at the first boundary (raypath.py:158, 179-180); every later one has
+        // nratio = 1 (raypath.py:257), which leaves the direction as it is
+        const double c = -dot(s, geo.n);                 // cos(t_inc)
+        const double nratio = Nl[0] / Nl[1];
+        const double st = nratio * sqrt(1.0 - c * c);    // sin(t_tran)
+        s = nratio * s + (nratio * c - sqrt(1.0 - st * st)) * geo.n;
+    }
+    // The rest of the path is the straight line r + t s, so a step is a chain in t alone: the
+    // point's y and |r|^2 (for f^2 at its latitude), r.s, the root of the next shell.  The next
+    // shell's radius is taken at the current point's latitude (raypath.py:182), hence
+    // disc = (r.s)^2 - f^2 (R_k^2 - R_{k+1}^2).  One thread's chain per ray bounds the kernel
+    // (carrying the point, two angles and four roots it took 0.48 us a step; as a chain in t
+    // 0.17 us: 1000 layers x 4 rays 480 -> 166 us, 800 layers x 16384 rays 440 -> 153 us).
+    double t = 0.0, y1 = r.y, q1 = dot(r, r), d1 = dot(r, s);
     int count = 0;
-    double rNow = geo.rmag;                           // shell layer at the current point
-    double rNext = ellipse(G, Rl[1], q).rmag;         // shell layer + 1 at the same latitude (raypath.py:182)
-    // equatorial radii of shells layer + 1 and layer + 2, the latter loaded a step ahead (its
-    // load latency hides behind one step of the chain)
-    double R1 = Rl[1], R2 = nl > 2 ? Rl[2] : 0.0;
-    while (true) {
-        s = nratio * s + (nratio * c - ct) * n;      // raypath.py:179-180 (ingress)
-        const double rdots = dot(r, s);
-        const double disc = rdots * rdots + rNext * rNext - rNow * rNow;
-        double ds = -rdots - sqrt(disc);             // NaN when the shell is missed
-        if (ds < 0.0) break;                         // raypath.py:212-216
-        if (A.limb == 1) ds = fabs(rNext - rNow) / mu;
-        out[count] = cm_half ? (ds * 1.0E3 / 1.0E-2) * 0.5 : ds;
-        ++count;
-        const V3 rn = r + ds * s;
-        double f;
-        shell_at(G, rn, f, n);
-        rNow = R1 * f;
-        r = rn;
-        ++layer;
-        c = -dot(s, n);
-        if (layer + 1 >= nl) break;                  // IndexError on nr[layer + 1]
-        rNext = R2 * f;
-        R1 = R2;
-        R2 = layer + 2 < nl ? Rl[layer + 2] : 0.0;
-        nratio = 1.0;
-        st = sqrt(1.0 - c * c);
-        ct = sqrt(1.0 - st * st);
+    double f2 = geo.rmag / rNorm;                        // the first step: at the edge's latitude
+    f2 *= f2;
+    // Equatorial radii by windows of kWin steps, the next window's loads issued a window ahead: a
+    // step is shorter than a load, and fetched one step ahead each step waited for one (1000
+    // layers x 4 rays 256 us).
+    // A lane whose path has ended computes on (nothing it writes): the window has no exits.
+    const double unit = A.units == 1 ? 5.0E4 : 1.0;      // half steps in cm, or km
+    double win[kWin + 1], nxt[kWin];
+#pragma unroll
+    for (int u = 0; u <= kWin; ++u) win[u] = Rl[min(u, nl - 1)];
+    bool alive = true;
+    for (int k0 = 0; alive; k0 += kWin) {
+#pragma unroll
+        for (int u = 0; u < kWin; ++u) nxt[u] = Rl[min(k0 + kWin + 1 + u, nl - 1)];
+#pragma unroll
+        for (int u = 0; u < kWin; ++u) {
+            const double R0 = win[u], R1 = win[u + 1];
+            const double rdots = d1 + t;
+            const double disc = fma(rdots, rdots, -f2 * ((R0 - R1) * (R0 + R1)));
+            double ds = -rdots - sqrt_km2(disc);         // NaN when the shell is missed
+            // the path ends below a shell (raypath.py:212-216) or at the last one (the
+            // IndexError on nr[layer + 1])
+            alive = alive && !(ds < 0.0) && k0 + u < nl - 1;
+            if constexpr (SEC) ds = fabs(R1 - R0) * sqrt(f2) / mu;
+            if (alive) out[k0 + u] = ds * unit;
+            count += alive ? 1 : 0;
+            t += ds;
+            const double y = fma(t, s.y, y1);
+            f2 = shell_f2(flat, y, fma(t, fma(2.0, d1, t), q1));
+            // incidence past 90 degrees, cos(t_inc) = -s.n < 0 with n along (ratio x, y, ratio z):
+            // the reference's arcsin(sin t_inc) then folds the angle, which turns the direction
+            // by 2 cos n
+            const double ys = y * s.y, along = fma(G.ratio, (d1 + t) - ys, ys);
+            if (__builtin_expect(alive && along > 0.0, 0)) {
+                r = r + t * s;
+                V3 n = {G.ratio * r.x, r.y, G.ratio * r.z};
+                n = (1.0 / norm(n)) * n;
+                const double c = -dot(s, n), st = sqrt(1.0 - c * c);
+                s = s + (c - sqrt(1.0 - st * st)) * n;
+                t = 0.0;
+                y1 = r.y;
+                q1 = dot(r, r);
+                d1 = dot(r, s);
+            }
+        }
+        win[0] = win[kWin];
+#pragma unroll
+        for (int u = 0; u < kWin; ++u) win[u + 1] = nxt[u];
     }
     A.nsteps[ray] = count;
 }
@@ -276,8 +321,11 @@ static int fill_ray_args(rbx::RayArgs &A, const rbx_planet *planet, const double
 
 static int launch_rays(const rbx::RayArgs &A, void *stream) {
     const int threads = rbx::kRayThreads;
-    hipLaunchKernelGGL(rbx::raypath_kernel, dim3((A.nray + threads - 1) / threads), dim3(threads), 0,
-                       static_cast<hipStream_t>(stream), A);
+    const dim3 grid((A.nray + threads - 1) / threads);
+    if (A.limb == 1)
+        hipLaunchKernelGGL(rbx::raypath_kernel<true>, grid, dim3(threads), 0, static_cast<hipStream_t>(stream), A);
+    else
+        hipLaunchKernelGGL(rbx::raypath_kernel<false>, grid, dim3(threads), 0, static_cast<hipStream_t>(stream), A);
     return rbx::launch_status("raypath_kernel");
 }
 
