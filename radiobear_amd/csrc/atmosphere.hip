@@ -1,9 +1,8 @@
 // Atmosphere construction on the device: computeProp's radii and refractive
 // indices (atm_base.py:120-181), optionally after a hydrostatic recomputation of
 // z, and its whole property table (atm_base.py:120-194), for many atmospheres laid
-// end to end.  One thread per atmosphere walks its layers (a few hundred steps of a
-// handful of FP64 operations); a retrieval batch of 1024 atmospheres is 16
-// wavefronts.
+// end to end.  Radii and indices: one block per atmosphere, a thread per layer.  The
+// property table: one thread per atmosphere walks its layers.
 #include "common.hpp"
 
 namespace rbx {
@@ -57,30 +56,82 @@ struct AtmArgs {
     double *Z, *R, *N;
 };
 
-__global__ __launch_bounds__(64) void atmosphere_kernel(AtmArgs A) {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= A.natm) return;
+constexpr int kAtmThreads = 256;
+
+// the block's nearest layer to p_ref (ref_layer: first of equals, l0 when none is within 1e6)
+__device__ inline int ref_layer_block(const double *P, int l0, int l1, double p_ref, double *dist, int *at) {
+    const int tid = threadIdx.x;
+    double best = 1.0E6;
+    int idx = 0x7fffffff;
+    for (int l = l0 + tid; l < l1; l += kAtmThreads) {
+        const double d = fabs(P[l] - p_ref);
+        if (d < best) {
+            best = d;
+            idx = l;
+        }
+    }
+    dist[tid] = best;
+    at[tid] = idx;
+    __syncthreads();
+    for (int s = kAtmThreads / 2; s > 0; s >>= 1) {
+        if (tid < s) {
+            const double d = dist[tid + s];
+            const int i = at[tid + s];
+            if (d < dist[tid] || (d == dist[tid] && i < at[tid])) {
+                dist[tid] = d;
+                at[tid] = i;
+            }
+        }
+        __syncthreads();
+    }
+    return at[0] == 0x7fffffff ? l0 : at[0];
+}
+
+// One block per atmosphere: the hydrostatic z is a running sum up from the deepest layer, taken
+// kAtmThreads layers at a time (a scan per wavefront, then over the wavefronts, plus the sum so
+// far).  One thread per atmosphere walked it serially, one log and two divisions a layer on one
+// lane of one CU: 64 atmospheres of 200-800 layers 1606 -> 13.8 us.
+__global__ __launch_bounds__(kAtmThreads) void atmosphere_kernel(AtmArgs A) {
+    __shared__ double dist[kAtmThreads];
+    __shared__ int at[kAtmThreads];
+    __shared__ double wsum[kAtmThreads / 64];
+    const int a = blockIdx.x, tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
     const int l0 = A.layer_off[a], l1 = A.layer_off[a + 1];
     if (l0 < 0 || l1 > A.nl_total || l1 - l0 < 1) return;   // bad offsets: rows left untouched
     const size_t nlt = A.nl_total;
     const double *P = A.P, *T = A.T;
     if (A.Zin) {
-        for (int l = l0; l < l1; ++l) A.Z[l] = A.Zin[l];
+        for (int l = l0 + tid; l < l1; l += kAtmThreads) A.Z[l] = A.Zin[l];
     } else {
         // hydrostatic z (km), deepest layer z = 0: dz = (H_i + H_{i+1})/2 ln(P_{i+1}/P_i),
         // H = R T / (m g) with one g for the atmosphere
-        double Hn = kRgas * T[l1 - 1] / (mean_amu(A.mix, nlt, l1 - 1) * A.g) / 1000.0;
-        double z = 0.0;
-        A.Z[l1 - 1] = 0.0;
-        for (int l = l1 - 2; l >= l0; --l) {
-            const double H = kRgas * T[l] / (mean_amu(A.mix, nlt, l) * A.g) / 1000.0;
-            z = z + 0.5 * (H + Hn) * log(P[l + 1] / P[l]);
-            A.Z[l] = z;
-            Hn = H;
+        auto scale_height = [&](int l) { return kRgas * T[l] / (mean_amu(A.mix, nlt, l) * A.g) / 1000.0; };
+        if (tid == 0) A.Z[l1 - 1] = 0.0;
+        double z0 = 0.0;   // z below this chunk
+        for (int c = l1 - 2; c >= l0; c -= kAtmThreads) {
+            const int l = c - tid;
+            double v = l >= l0 ? 0.5 * (scale_height(l) + scale_height(l + 1)) * log(P[l + 1] / P[l]) : 0.0;
+#pragma unroll
+            for (int m = 1; m < 64; m <<= 1) {
+                const double y = __shfl_up(v, m);
+                if (lane >= m) v += y;
+            }
+            if (lane == 63) wsum[wave] = v;
+            __syncthreads();
+            double below = z0, all = z0;
+#pragma unroll
+            for (int w = 0; w < kAtmThreads / 64; ++w) {
+                if (w < wave) below += wsum[w];
+                all += wsum[w];
+            }
+            if (l >= l0) A.Z[l] = below + v;
+            z0 = all;
+            __syncthreads();   // (the next chunk overwrites wsum)
         }
     }
-    const double zoff = A.Z[ref_layer(P, l0, l1, A.p_ref)];
-    for (int l = l0; l < l1; ++l) {
+    const int iref = ref_layer_block(P, l0, l1, A.p_ref, dist, at);   // (its barriers order the writes of Z)
+    const double zoff = A.Z[iref];
+    for (int l = l0 + tid; l < l1; l += kAtmThreads) {
         A.R[l] = A.req + A.Z[l] - zoff;                                               // atm_base.py:147
         A.N[l] = refractivity(A.mix, nlt, l, T[l]) * P[l] * (293.0 / T[l]) / 1.0E6 + 1.0;   // atm_base.py:176-181
     }
@@ -189,7 +240,7 @@ extern "C" int rbx_atmosphere_batch(const double *P, const double *T, const doub
     A.Z = Z;
     A.R = R;
     A.N = N;
-    hipLaunchKernelGGL(rbx::atmosphere_kernel, dim3((natm + 63) / 64), dim3(64), 0,
+    hipLaunchKernelGGL(rbx::atmosphere_kernel, dim3(natm), dim3(rbx::kAtmThreads), 0,
                        static_cast<hipStream_t>(stream), A);
     return rbx::launch_status("atmosphere_kernel");
 }
