@@ -1312,19 +1312,26 @@ __device__ inline void put_prep(double *row, const P &p) {
     for (int k = 0; k < prep_words<P>(); ++k) row[k] = w[k];
 }
 
-__global__ __launch_bounds__(256) void tangent_prep_kernel(AlphaArgs A) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= A.nl * kTanSegs) return;
-    const int layer = e / kTanSegs, seg = e % kTanSegs;
+// (derivers slowest, a wavefront per block, as alpha_prep_kernel: 32000 layers 53 -> 27 us, 500
+// layers 33 -> 12 us)
+constexpr int kTanPrepThreads = 64;
+constexpr int kTanDerivers = kTanSegs + 1;   // kTanSegs: the inversion lines' set 1
+__global__ __launch_bounds__(kTanPrepThreads) void tangent_prep_kernel(AlphaArgs A) {
+    const long long e = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (e >= static_cast<long long>(A.nl) * kTanDerivers) return;
+    const int layer = static_cast<int>(e % A.nl), which = static_cast<int>(e / A.nl);
+    const int seg = which == kTanSegs ? 2 : which;
     const LayerT<Dual> L = dual_layer(A, layer);
     double *row = A.tan_prep + static_cast<size_t>(layer) * kTanPrepWords + kTanPrepOff[seg];
-    switch (seg) {
+    switch (which) {
         case 0: put_prep(row, H2oPrep<Dual>(L)); break;
         case 1: put_prep(row, H2sPrep<Dual>(L)); break;
         case 2:
-            put_prep(row, InvPrep<Dual>(L, nh3_low_set(A.abs.nh3)));
-            put_prep(row + prep_words<InvPrep<Dual>>(), InvPrep<Dual>(L, 1));
+        case kTanSegs: {
+            const int s = which == kTanSegs ? 1 : 0;
+            put_prep(row + s * prep_words<InvPrep<Dual>>(), InvPrep<Dual>(L, s ? 1 : nh3_low_set(A.abs.nh3)));
             break;
+        }
         case 3: put_prep(row, RotPrep<Dual>(L)); break;
         case 4: put_prep(row, V2Prep<Dual>(L)); break;
         default: put_prep(row, Ph3Prep<Dual>(L)); break;
@@ -1766,8 +1773,9 @@ static int launch_alpha(AlphaArgs &A, int precision, int nsplit, hipStream_t st)
 template <int K, bool F32>
 static int launch_series(AlphaArgs &A, hipStream_t st) {
     const long long groups = (A.tiles_total + kFarTiles - 1) / kFarTiles;
-    hipLaunchKernelGGL(alpha_prep_kernel<F32>, dim3(static_cast<unsigned>((static_cast<long long>(A.nl) * kSegs + 255) / 256)),
-                       dim3(256), 0, st, A);
+    hipLaunchKernelGGL(alpha_prep_kernel<F32>,
+                       dim3(static_cast<unsigned>((static_cast<long long>(A.nl) * kPrepDerivers + kPrepThreads - 1) / kPrepThreads)),
+                       dim3(kPrepThreads), 0, st, A);
     int rc = launch_status("alpha_prep_kernel");
     if (rc) return rc;
     dim3 g1(static_cast<unsigned>(groups * A.nl), static_cast<unsigned>(A.far_split));
@@ -2083,8 +2091,10 @@ extern "C" int rbx_alpha_tangent(const rbx_catalog *cat, const rbx_absorbers *ab
     hipStream_t st = static_cast<hipStream_t>(stream);
     const dim3 gs(static_cast<unsigned>(groups), static_cast<unsigned>(std::max(parts, 1))), bs(64 * W);
     const bool f32 = precision == RBX_FP32;
-    hipLaunchKernelGGL(rbx::tangent_prep_kernel, dim3(static_cast<unsigned>((static_cast<long long>(nl) * rbx::kTanSegs + 255) / 256)),
-                       dim3(256), 0, st, A);
+    hipLaunchKernelGGL(rbx::tangent_prep_kernel,
+                       dim3(static_cast<unsigned>((static_cast<long long>(nl) * rbx::kTanDerivers + rbx::kTanPrepThreads - 1) /
+                                                  rbx::kTanPrepThreads)),
+                       dim3(rbx::kTanPrepThreads), 0, st, A);
     rc = rbx::launch_status("tangent_prep_kernel");
     if (rc) return rc;
 #define RBX_TAN_LAUNCH(MODE)                                                                                    \

@@ -20,7 +20,7 @@
 // the same 16 terms at ratio 0.15 (at most ~8e-12 of a far line's value) and sums its near
 // lines in FP64 from their (D, a, c, g, G), as the direct FP64 sums do.
 //
-// alpha_prep_kernel (one thread per layer and segment) first writes every layer's
+// alpha_prep_kernel (one thread per layer and deriver) first writes every layer's
 // coefficient derivers to the workspace; both passes below read them from there.
 // alpha_far_kernel (block = layer x group of kFarTiles tiles x part of the layer's
 // staging rounds; each wavefront a contiguous run of 64-line blocks): each lane derives
@@ -139,58 +139,48 @@ constexpr int kPrepWords = 18;
 template <int S>
 using SegC = std::integral_constant<int, S>;
 
+// One thread per (deriver, layer), derivers slowest: the lanes of a wavefront build the same
+// deriver (with the layer slowest they ran all six one after the other), and the nh3_hs inversion
+// lines' two sets are two derivers.  A wavefront per block spreads the few of them over the CUs.
+// The powers' latency bounds it: 800 layers 20 -> 9 us, 400 layers 22 -> 9 us.
+constexpr int kPrepThreads = 64;
+constexpr int kPrepDerivers = kSegs + 1;   // kSegs: the inversion lines' set 1
+
 template <bool F32>
-__global__ __launch_bounds__(256) void alpha_prep_kernel(AlphaArgs A) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= A.nl * kSegs) return;
-    const int layer = e / kSegs, seg = e % kSegs;
+__global__ __launch_bounds__(kPrepThreads) void alpha_prep_kernel(AlphaArgs A) {
+    const long long e = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (e >= static_cast<long long>(A.nl) * kPrepDerivers) return;
+    const int layer = static_cast<int>(e % A.nl), which = static_cast<int>(e / A.nl);
+    const int seg = which == kSegs ? 2 : which;
     const LayerT<double> L = layer_of(A, layer);
     const DevBlock *blk = A.cat.blk;
-    double *row = A.far_prep + static_cast<size_t>(e) * kPrepWords;
-    auto put = [&](const auto &p0, const auto &p1, double s0, double s1) {
-        using Prep = std::decay_t<decltype(p0)>;
+    double *row = A.far_prep + (static_cast<size_t>(layer) * kSegs + seg) * kPrepWords;
+    // the deriver into set s's words, its weight scale into word 16 + s
+    auto put = [&](int s, const auto &p, double sc) {
+        using Prep = std::decay_t<decltype(p)>;
         static_assert(sizeof(Prep) <= 8 * sizeof(double) && sizeof(Prep) % sizeof(double) == 0,
                       "a deriver is at most 8 doubles");
-        const double *w0 = reinterpret_cast<const double *>(&p0), *w1 = reinterpret_cast<const double *>(&p1);
-        for (int k = 0; k < 8; ++k) {
-            row[k] = k < static_cast<int>(sizeof(Prep) / sizeof(double)) ? w0[k] : 0.0;
-            row[8 + k] = k < static_cast<int>(sizeof(Prep) / sizeof(double)) ? w1[k] : 0.0;
-        }
-        row[16] = F32 ? s0 : 1.0;
-        row[17] = F32 ? s1 : 1.0;
+        const double *w = reinterpret_cast<const double *>(&p);
+        for (int k = 0; k < 8; ++k) row[8 * s + k] = k < static_cast<int>(sizeof(Prep) / sizeof(double)) ? w[k] : 0.0;
+        row[16 + s] = F32 ? sc : 1.0;
     };
-    switch (seg) {
-        case 0: {
-            const H2oPrep<double> p(L);
-            put(p, p, pow2_scale(p.pref * blk[RBX_LINES_H2O].wscale), 1.0);
+    auto one = [&](const auto &p, int kind) {   // segments of one set: both halves the same
+        put(0, p, pow2_scale(p.pref * blk[kind].wscale));
+        put(1, p, 1.0);
+    };
+    switch (which) {
+        case 0: one(H2oPrep<double>(L), RBX_LINES_H2O); break;
+        case 1: one(H2sPrep<double>(L), RBX_LINES_H2S); break;
+        case 2:
+        case kSegs: {
+            const int s = which == kSegs ? 1 : 0;
+            const InvPrep<double> p(L, s ? 1 : nh3_low_set(A.abs.nh3));
+            put(s, p, pow2_scale(p.pref * blk[RBX_LINES_NH3_INV].wscale));
             break;
         }
-        case 1: {
-            const H2sPrep<double> p(L);
-            put(p, p, pow2_scale(p.pref * blk[RBX_LINES_H2S].wscale), 1.0);
-            break;
-        }
-        case 2: {
-            const InvPrep<double> p0(L, nh3_low_set(A.abs.nh3)), p1(L, 1);
-            const double w = blk[RBX_LINES_NH3_INV].wscale;
-            put(p0, p1, pow2_scale(p0.pref * w), pow2_scale(p1.pref * w));
-            break;
-        }
-        case 3: {
-            const RotPrep<double> p(L);
-            put(p, p, pow2_scale(p.pref * blk[RBX_LINES_NH3_ROT].wscale), 1.0);
-            break;
-        }
-        case 4: {
-            const V2Prep<double> p(L);
-            put(p, p, pow2_scale(p.pref * blk[RBX_LINES_NH3_V2].wscale), 1.0);
-            break;
-        }
-        default: {
-            const Ph3Prep<double> p(L);
-            put(p, p, pow2_scale(p.pref * blk[RBX_LINES_PH3].wscale), 1.0);
-            break;
-        }
+        case 3: one(RotPrep<double>(L), RBX_LINES_NH3_ROT); break;
+        case 4: one(V2Prep<double>(L), RBX_LINES_NH3_V2); break;
+        default: one(Ph3Prep<double>(L), RBX_LINES_PH3); break;
     }
 }
 
