@@ -1,4 +1,4 @@
-// Ray geometry in FP64: one thread per ray.
+// Ray geometry in FP64: a ray's steps split over 32 lanes, or one thread per ray.
 //
 // Follows raypath.compute_ds / findEdge (raypath.py:60-273) and the ellipse
 // branch of Shape (shape.py:223-298) step for step.  The reference converts
@@ -112,13 +112,15 @@ __device__ inline double shell_f2(double flat, double y, double q) {
     return fma(-flat, s2, 1.0);
 }
 
-// Rays per block.  One thread per ray: a ray's path is one dependent chain of FP64 steps, so
-// the kernel is latency-bound and holds few wavefronts (256 for 16384 rays).  It runs beside the
-// line sums (rbx_alpha) when a caller puts it on a second stream or graph branch; four
-// wavefronts per block keep it on a quarter as many CUs as one per block, leaving the other
-// CUs' slots whole for the line sums: 800 layers x 1024 frequencies x 16384 rays, graph step
-// 3.71 -> 3.47 ms when the paths alone took 0.42 -> 0.45 ms (2 and 8 wavefronts per block: 3.59,
-// 3.53 ms).
+// The direction after incidence past 90 degrees at r: the reference's arcsin(sin t_inc) folds the
+// angle, which turns the direction by 2 cos n (n along (ratio x, y, ratio z)).
+__device__ inline V3 reflected(const Geo &G, V3 r, V3 s) {
+    V3 n = {G.ratio * r.x, r.y, G.ratio * r.z};
+    n = (1.0 / norm(n)) * n;
+    const double c = -dot(s, n), st = sqrt(1.0 - c * c);
+    return s + (c - sqrt(1.0 - st * st)) * n;
+}
+
 constexpr int kRayThreads = 256;
 constexpr int kWin = 8;   // shell radii fetched per window
 
@@ -139,10 +141,179 @@ struct RayArgs {
     int natm;
 };
 
+// A path from point r along s (any |s|^2 = 1) over the shells from `step` on, step by step: the
+// path is the straight line r + t s, so a step is a chain in t alone: the point's y and |r|^2
+// (for f^2 at its latitude), r.s, the root of the next shell.  The next shell's radius is taken
+// at the current point's latitude (raypath.py:182), hence disc = (r.s)^2 - f^2 (R_k^2 - R_{k+1}^2).
+// f2: f^2 for the first of the steps.  Returns the step count; `write`: this lane writes the steps.
+// One step's chain is 0.17 us (it was 0.48 us carrying the point, two angles and four roots).
 // SEC: limb 'sec' (raypath.py:218-219)
 template <bool SEC>
+__device__ inline int serial_steps(const RayArgs &A, const double *Rl, int nl, double *out, double flat, double unit,
+                                   double mu, V3 r, V3 s, double f2, int step, bool write) {
+    const Geo &G = A.G;
+    double t = 0.0, y1 = r.y, q1 = dot(r, r), d1 = dot(r, s);
+    int count = step;
+    // Equatorial radii by windows of kWin steps, the next window's loads issued a window ahead: a
+    // step is shorter than a load, and fetched one step ahead each step waited for one (1000
+    // layers x 4 rays 256 us against 166 us).
+    // A lane whose path has ended computes on (nothing it writes): the window has no exits.
+    double win[kWin + 1], nxt[kWin];
+#pragma unroll
+    for (int u = 0; u <= kWin; ++u) win[u] = Rl[min(step + u, nl - 1)];
+    bool alive = true;
+    for (int k0 = step; alive; k0 += kWin) {
+#pragma unroll
+        for (int u = 0; u < kWin; ++u) nxt[u] = Rl[min(k0 + kWin + 1 + u, nl - 1)];
+#pragma unroll
+        for (int u = 0; u < kWin; ++u) {
+            const double R0 = win[u], R1 = win[u + 1];
+            const double rdots = d1 + t;
+            const double disc = fma(rdots, rdots, -f2 * ((R0 - R1) * (R0 + R1)));
+            double ds = -rdots - sqrt_km2(disc);         // NaN when the shell is missed
+            // the path ends below a shell (raypath.py:212-216) or at the last one (the
+            // IndexError on nr[layer + 1])
+            alive = alive && !(ds < 0.0) && k0 + u < nl - 1;
+            if constexpr (SEC) ds = fabs(R1 - R0) * sqrt(f2) / mu;
+            if (alive && write) out[k0 + u] = ds * unit;
+            count += alive ? 1 : 0;
+            t += ds;
+            const double y = fma(t, s.y, y1);
+            f2 = shell_f2(flat, y, fma(t, fma(2.0, d1, t), q1));
+            // incidence past 90 degrees, cos(t_inc) = -s.n < 0 with n along (ratio x, y, ratio z)
+            const double ys = y * s.y, along = fma(G.ratio, (d1 + t) - ys, ys);
+            if (__builtin_expect(alive && along > 0.0, 0)) {
+                r = r + t * s;
+                s = reflected(G, r, s);
+                t = 0.0;
+                y1 = r.y;
+                q1 = dot(r, r);
+                d1 = dot(r, s);
+            }
+        }
+        win[0] = win[kWin];
+#pragma unroll
+        for (int u = 0; u < kWin; ++u) win[u + 1] = nxt[u];
+    }
+    return count;
+}
+
+// The same path by L lanes, each a run of consecutive steps.  With u_k = |r_k|^2 - |r_0|^2 a step
+// is u_{k+1} = u_k - f^2(u_k) (R_k^2 - R_{k+1}^2), -r_k.s = S_k = sqrt((r_0.s)^2 + u_k) on the way
+// in, and ds_k = (u_k - u_{k+1}) / (S_k + S_{k+1}).  f^2 changes slowly along a path, so lane c
+// starts from a guess of its first u, walks its run, and tracks d(its last u)/d(its first u): the
+// runs' affine maps composed over the lanes (a scan) give every lane a better first u.  The walk is
+// repeated until no first u moves; each pass makes at least one more run exact, so L + 1 always
+// suffice, and away from the limb 2 or 3 do.  Where a shell is missed, S and ds are NaN from there
+// on, as in the serial steps.  Returns the step count, or -1 - k when the path meets incidence past
+// 90 degrees at step k (reached with S in S_at): the caller goes on from there step by step.
+template <int L>
+__device__ inline int parallel_steps(const RayArgs &A, const double *Rl, int nl, double *out, double flat,
+                                     double unit, V3 r, V3 s, double f2_first, int c, double (*stage)[kWin],
+                                     double &S_at) {
+    constexpr int W = kWin;
+    const double ratio = A.G.ratio, sy = s.y, y1 = r.y, q1 = dot(r, r), d1 = dot(r, s), d1sq = d1 * d1;
+    const int n = nl - 1, len = (n + L - 1) / L;
+    const int kb = min(n, c * len), ke = min(n, kb + len);
+    const int lane0 = (threadIdx.x % 64) / L * L;
+    const unsigned long long group = (L == 64 ? ~0ull : ((1ull << (L % 64)) - 1ull)) << lane0;
+    double u0 = 0.0;
+    if (c > 0) {   // du/dB = -f^2(u) to second order in B = R_0^2 - R_k^2, the first step's own f^2 apart
+        const double Ra = Rl[0], Rb = Rl[kb], R1 = Rl[1];
+        const double B = (Ra - Rb) * (Ra + Rb), f = shell_f2(flat, y1, q1);
+        const double g = flat * (y1 / q1) * (y1 / q1 - sy / d1);
+        u0 = fma(-f, B, 0.5 * f * g * B * B) - (f2_first - f) * ((Ra - R1) * (Ra + R1));
+    }
+    int neg = n, refl = n;   // first step with ds < 0, first point past 90 degrees
+    for (int pass = 0; pass <= L + 1; ++pass) {
+        double u = u0, S = sqrt_km2(d1sq + u0), D = 1.0;
+        double S_r = 0.0;
+        neg = refl = n;
+        double win[W + 1], nxt[W];
+#pragma unroll
+        for (int i = 0; i <= W; ++i) win[i] = Rl[min(kb + i, n)];
+        for (int off = 0; off < len; off += W) {   // (the same trips for the ray's lanes)
+            const int k0 = kb + off;
+#pragma unroll
+            for (int i = 0; i < W; ++i) nxt[i] = Rl[min(k0 + W + 1 + i, n)];
+#pragma unroll
+            for (int i = 0; i < W; ++i) {
+                const int k = k0 + i;
+                if (k < ke) {
+                    const double y = fma(-(S + d1), sy, y1), q = q1 + u, ys = y * sy;
+                    const double iq = rcp_pos(q);
+                    const double f2 = k == 0 ? f2_first : fma(-flat, y == 0.0 ? kLat0 : y * y * iq, 1.0);
+                    if (k > 0 && refl == n && fma(ratio, -S - ys, ys) > 0.0) {
+                        refl = k;
+                        S_r = S;
+                    }
+                    const double dR = (win[i] - win[i + 1]) * (win[i] + win[i + 1]);
+                    const double v = f2 * dR, un = u - v, Sn = sqrt_km2(d1sq + un);
+                    const double ds = v * rcp_pos(S + Sn);
+                    if (neg == n && ds < 0.0) neg = k;
+                    stage[c][i] = ds * unit;
+                    // 1 - d f^2/du dR (a derivative: the estimate of 1 / S will do)
+                    D *= fma(-flat * dR * iq, fma(ys, __builtin_amdgcn_rcp(S), y * y * iq), 1.0);
+                    u = un;
+                    S = Sn;
+                }
+            }
+            win[0] = win[W];
+#pragma unroll
+            for (int i = 0; i < W; ++i) win[i + 1] = nxt[i];
+            // the window's steps leave through LDS: L consecutive lanes write whole pieces of the
+            // lanes' runs (each lane writing its own step touches one line per lane and store).  The
+            // first pass, a guess, writes nothing.
+            if (pass > 0) {
+                wave_sync();
+#pragma unroll
+                for (int j = 0; j < W; ++j) {
+                    const int e = j * L + c, o = e / W, k = o * len + off + e % W;
+                    if (off + e % W < len && k < n) out[k] = stage[o][e % W];
+                }
+                wave_sync();
+            }
+        }
+        // how far lane c's first u moves: the end of the run before it against it, plus what the
+        // moves of earlier runs do to that end (a difference, so that settled runs leave no noise)
+        const bool bad = __builtin_isnan(u0);
+        double e = __shfl_up(u, 1, L) - (bad ? 0.0 : u0), Dp = __shfl_up(D, 1, L);
+        if (c == 0) e = Dp = 0.0;
+#pragma unroll
+        for (int m = 1; m < L; m <<= 1) {
+            const double em = __shfl_up(e, m, L), Dm = __shfl_up(Dp, m, L);
+            if (c >= m) {
+                e = fma(Dp, em, e);
+                Dp *= Dm;
+            }
+        }
+        const double next = (bad ? 0.0 : u0) + e, w = d1sq + next;
+        const bool missed = !(w >= 0.0) && !(d1sq + u0 >= 0.0);   // NaN steps before and after
+        const bool settled = c == 0 || kb >= ke || missed ||
+                             (!bad && fabs(e) <= 1.0e-13 * fabs(w) + 1.0e-15 * fabs(next));
+        S_at = S_r;
+        if (pass > 0 && (__builtin_amdgcn_ballot_w64(!settled) & group) == 0ull) break;
+        if (c > 0) u0 = next;
+    }
+    int first = refl, at = neg;
+#pragma unroll
+    for (int m = 1; m < L; m <<= 1) {
+        first = min(first, __shfl_xor(first, m, L));
+        at = min(at, __shfl_xor(at, m, L));
+    }
+    if (first < at) {
+        S_at = __shfl(S_at, first / len, L);
+        return -1 - first;
+    }
+    return at;
+}
+
+// L lanes per ray (1: a thread walks its ray's steps).
+template <bool SEC, int L>
 __global__ __launch_bounds__(kRayThreads) void raypath_kernel(RayArgs A) {
-    const int ray = blockIdx.x * blockDim.x + threadIdx.x;
+    __shared__ double stage[L > 1 ? kRayThreads : 1][kWin];
+    const long long id = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int ray = static_cast<int>(id / L), c = static_cast<int>(id % L);
     if (ray >= A.nray) return;
     const double b0 = A.b[2 * ray], b1 = A.b[2 * ray + 1];
     double *out = A.ds + static_cast<size_t>(ray) * A.ld;
@@ -154,7 +325,7 @@ __global__ __launch_bounds__(kRayThreads) void raypath_kernel(RayArgs A) {
         const int l0 = (a >= 0 && a < A.natm) ? A.layer_off[a] : -1;
         const int l1 = (a >= 0 && a < A.natm) ? A.layer_off[a + 1] : -1;
         if (l0 < 0 || l1 > A.nl || l1 - l0 < 2 || l1 - l0 - 1 > A.ld) {   // bad index or offsets
-            A.nsteps[ray] = -2;
+            if (c == 0) A.nsteps[ray] = -2;
             return;
         }
         Rl += l0;
@@ -164,7 +335,7 @@ __global__ __launch_bounds__(kRayThreads) void raypath_kernel(RayArgs A) {
     const double rNorm = Rl[0];
     const double tmp = b0 * b0 + b1 * b1;
     if (!(tmp < 1.0)) {                                // raypath.py:126-127 (NaN b: off planet too)
-        A.nsteps[ray] = -1;
+        if (c == 0) A.nsteps[ray] = -1;
         return;
     }
     const double mu = sqrt(1.0 - tmp);
@@ -179,17 +350,22 @@ __global__ __launch_bounds__(kRayThreads) void raypath_kernel(RayArgs A) {
     const double flat = 1.0 - G.ratio * G.ratio;
     auto trial = [&](int i) { return (i == 0) ? start : ((i == 1) ? z1 : start + i * dz); };
     int hit = -1;
-    for (int i = 0; i < ntrial; ++i) {
+    for (int i0 = 0; i0 < ntrial && hit < 0; i0 += L) {   // L trials at a time, the first below taken
+        const int i = i0 + c;
         const V3 bv = mat(G.M, V3{b0, b1, trial(i)});
         const double q = dot(bv, bv), Y = bv.y * bv.y;
         // q < f^2 times q > 0 (1e-6 rad at y == 0)
-        if (q * q < fma(-flat, bv.y == 0.0 ? kLat0 * q : Y, q)) {
-            hit = i;
-            break;
+        const bool below = i < ntrial && q * q < fma(-flat, bv.y == 0.0 ? kLat0 * q : Y, q);
+        if constexpr (L == 1) {
+            if (below) hit = i;
+        } else {
+            const unsigned long long any =
+                (__builtin_amdgcn_ballot_w64(below) >> (threadIdx.x % 64 / L * L)) & (~0ull >> (64 - L));
+            if (any != 0ull) hit = i0 + __builtin_ctzll(any);
         }
     }
     if (hit < 0) {
-        A.nsteps[ray] = -1;
+        if (c == 0) A.nsteps[ray] = -1;
         return;
     }
     auto above = [&](double z) {   // |v| - top shell radius at v's latitude
@@ -217,69 +393,32 @@ __global__ __launch_bounds__(kRayThreads) void raypath_kernel(RayArgs A) {
     {
         // refraction at the first boundary (raypath.py:158, 179-180); every later one has
         // nratio = 1 (raypath.py:257), which leaves the direction as it is
-        const double c = -dot(s, geo.n);                 // cos(t_inc)
+        const double ci = -dot(s, geo.n);                // cos(t_inc)
         const double nratio = Nl[0] / Nl[1];
-        const double st = nratio * sqrt(1.0 - c * c);    // sin(t_tran)
-        s = nratio * s + (nratio * c - sqrt(1.0 - st * st)) * geo.n;
+        const double st = nratio * sqrt(1.0 - ci * ci);  // sin(t_tran)
+        s = nratio * s + (nratio * ci - sqrt(1.0 - st * st)) * geo.n;
     }
-    // The rest of the path is the straight line r + t s, so a step is a chain in t alone: the
-    // point's y and |r|^2 (for f^2 at its latitude), r.s, the root of the next shell.  The next
-    // shell's radius is taken at the current point's latitude (raypath.py:182), hence
-    // disc = (r.s)^2 - f^2 (R_k^2 - R_{k+1}^2).  One thread's chain per ray bounds the kernel
-    // (carrying the point, two angles and four roots it took 0.48 us a step; as a chain in t
-    // 0.17 us: 1000 layers x 4 rays 480 -> 166 us, 800 layers x 16384 rays 440 -> 153 us).
-    double t = 0.0, y1 = r.y, q1 = dot(r, r), d1 = dot(r, s);
-    int count = 0;
     double f2 = geo.rmag / rNorm;                        // the first step: at the edge's latitude
     f2 *= f2;
-    // Equatorial radii by windows of kWin steps, the next window's loads issued a window ahead: a
-    // step is shorter than a load, and fetched one step ahead each step waited for one (1000
-    // layers x 4 rays 256 us).
-    // A lane whose path has ended computes on (nothing it writes): the window has no exits.
     const double unit = A.units == 1 ? 5.0E4 : 1.0;      // half steps in cm, or km
-    double win[kWin + 1], nxt[kWin];
-#pragma unroll
-    for (int u = 0; u <= kWin; ++u) win[u] = Rl[min(u, nl - 1)];
-    bool alive = true;
-    for (int k0 = 0; alive; k0 += kWin) {
-#pragma unroll
-        for (int u = 0; u < kWin; ++u) nxt[u] = Rl[min(k0 + kWin + 1 + u, nl - 1)];
-#pragma unroll
-        for (int u = 0; u < kWin; ++u) {
-            const double R0 = win[u], R1 = win[u + 1];
-            const double rdots = d1 + t;
-            const double disc = fma(rdots, rdots, -f2 * ((R0 - R1) * (R0 + R1)));
-            double ds = -rdots - sqrt_km2(disc);         // NaN when the shell is missed
-            // the path ends below a shell (raypath.py:212-216) or at the last one (the
-            // IndexError on nr[layer + 1])
-            alive = alive && !(ds < 0.0) && k0 + u < nl - 1;
-            if constexpr (SEC) ds = fabs(R1 - R0) * sqrt(f2) / mu;
-            if (alive) out[k0 + u] = ds * unit;
-            count += alive ? 1 : 0;
-            t += ds;
-            const double y = fma(t, s.y, y1);
-            f2 = shell_f2(flat, y, fma(t, fma(2.0, d1, t), q1));
-            // incidence past 90 degrees, cos(t_inc) = -s.n < 0 with n along (ratio x, y, ratio z):
-            // the reference's arcsin(sin t_inc) then folds the angle, which turns the direction
-            // by 2 cos n
-            const double ys = y * s.y, along = fma(G.ratio, (d1 + t) - ys, ys);
-            if (__builtin_expect(alive && along > 0.0, 0)) {
-                r = r + t * s;
-                V3 n = {G.ratio * r.x, r.y, G.ratio * r.z};
-                n = (1.0 / norm(n)) * n;
-                const double c = -dot(s, n), st = sqrt(1.0 - c * c);
-                s = s + (c - sqrt(1.0 - st * st)) * n;
-                t = 0.0;
-                y1 = r.y;
-                q1 = dot(r, r);
-                d1 = dot(r, s);
+    int step = 0;
+    if constexpr (L > 1) {
+        if (dot(r, s) < 0.0) {
+            double S;
+            const int got = parallel_steps<L>(A, Rl, nl, out, flat, unit, r, s, f2, c, stage + (threadIdx.x - c), S);
+            if (got >= 0) {
+                if (c == 0) A.nsteps[ray] = got;
+                return;
             }
+            step = -1 - got;
+            const double t = -S - dot(r, s);
+            r = r + t * s;
+            f2 = shell_f2(flat, r.y, dot(r, r));
+            s = reflected(G, r, s);
         }
-        win[0] = win[kWin];
-#pragma unroll
-        for (int u = 0; u < kWin; ++u) win[u + 1] = nxt[u];
     }
-    A.nsteps[ray] = count;
+    const int count = serial_steps<SEC>(A, Rl, nl, out, flat, unit, mu, r, s, f2, step, c == 0);
+    if (c == 0) A.nsteps[ray] = count;
 }
 
 }  // namespace rbx
@@ -319,13 +458,23 @@ static int fill_ray_args(rbx::RayArgs &A, const rbx_planet *planet, const double
     return RBX_OK;
 }
 
+// Lanes per ray: a thread's chain of steps bounds a launch until its wavefronts fill the SIMDs, so a
+// ray's steps are split over kRayLanes; past kSplitRays rays a thread per ray fills the device and
+// the second walk over the steps only adds work.  One number of lanes up to there, so that a ray's
+// path does not depend on the rays beside it.  Measured (us, 1 lane and 32): 1000 layers x 4 rays
+// 183 -> 23, 500 x 256 100 -> 22, 400 x 4096 82 -> 23, 800 x 16384 150 -> 93, 800 x 32768 176 -> 173,
+// 800 x 65536 233 against 330 (16 lanes 36, 24, 24, 87, 161, 298; 64 lanes 22, 21, 26, 106, 195).
+constexpr int kRayLanes = 32, kSplitRays = 32768;
+
 static int launch_rays(const rbx::RayArgs &A, void *stream) {
     const int threads = rbx::kRayThreads;
-    const dim3 grid((A.nray + threads - 1) / threads);
-    if (A.limb == 1)
-        hipLaunchKernelGGL(rbx::raypath_kernel<true>, grid, dim3(threads), 0, static_cast<hipStream_t>(stream), A);
-    else
-        hipLaunchKernelGGL(rbx::raypath_kernel<false>, grid, dim3(threads), 0, static_cast<hipStream_t>(stream), A);
+    const bool split = A.limb != 1 && A.nray <= kSplitRays;   // ('sec' steps leave the straight line)
+    const long long lanes = static_cast<long long>(A.nray) * (split ? kRayLanes : 1);
+    const dim3 grid(static_cast<unsigned>((lanes + threads - 1) / threads));
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (split) hipLaunchKernelGGL((rbx::raypath_kernel<false, kRayLanes>), grid, dim3(threads), 0, st, A);
+    else if (A.limb == 1) hipLaunchKernelGGL((rbx::raypath_kernel<true, 1>), grid, dim3(threads), 0, st, A);
+    else hipLaunchKernelGGL((rbx::raypath_kernel<false, 1>), grid, dim3(threads), 0, st, A);
     return rbx::launch_status("raypath_kernel");
 }
 
