@@ -177,7 +177,9 @@ typedef struct rbx_launch {
                            model of the grid's last dispatch wave) */
     int far_split;      /* parts each layer's lines are split into in the series' classification
                            pass: 1..16 (built in: about 4096 blocks) */
-    int int_unroll;     /* path steps per load batch of the integration: 4 or 8 (built in: 8) */
+    int int_unroll;     /* path steps per load batch of the integration: 4 or 8 (built in: 8;
+                           requests of few rays and frequencies split a ray's steps over
+                           threads instead, unless int_unroll or int_map is given) */
     int int_map;        /* integration block order: 1 frequency group major (each XCD keeps a
                            slice of the table for every ray), 2 ray major (each XCD runs every
                            frequency group of its rays: their ds rows are read once per ray and

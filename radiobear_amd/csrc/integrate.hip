@@ -412,6 +412,111 @@ __global__ __launch_bounds__(kWaves * kLanes) void integrate_f32_kernel(IntArgs 
     if (A.intW) A.intW[o] = (S < 0) ? 0.0 : intW;
 }
 
+// ---- few rays: a ray's steps split over segments ----
+// A wavefront's walk down a path is one dependent chain (a load batch, an FP64 add and an
+// exponential per step; an E2 per step for a disc), so a request of few (ray, 64 frequencies)
+// wavefronts is bound by that chain's latency with most of the chip idle: 112 us for 1000 layers
+// x 4 rays x 6 frequencies, 400-460 us for a disc of 150 layers x 20 frequencies (here 11 and 22 us:
+// the loads' latency, and one E2 a thread).  Here a block
+// takes COLS columns of one ray and its threads are SEGS runs of consecutive path points: each
+// thread adds its run's tau increments, a scan over the runs (shuffles, then the wavefronts'
+// totals through LDS) gives the tau a run starts from, and each thread then walks its run
+// exactly.  The two sums are taken by path point,
+// sum_i (W_i + W_{i+1}) h_i = sum_p W_p (h_{p-1} + h_p) (W_0 = 0, h_n = 0), so a run needs
+// nothing of its neighbours but the starting tau.  All FP64, also where the table is FP32.  The
+// tau cut ends each thread's walk at the first point past it.
+constexpr int kSegThreads = 1024;
+template <class AT, int MODE, int COLS>
+__global__ __launch_bounds__(kSegThreads) void integrate_segments_kernel(IntArgs A, int colgroups) {
+    constexpr int SEGS = kSegThreads / COLS, W = kSegThreads / kLanes;
+    __shared__ double etab[kExpTab];
+    __shared__ double part[2][W][COLS];
+    const int col = threadIdx.x % COLS, seg = threadIdx.x / COLS;
+    const int wave = threadIdx.x / kLanes, lane = threadIdx.x % kLanes;
+    if (MODE == 0 && threadIdx.x < kExpTab) etab[threadIdx.x] = kExp2Tab[threadIdx.x];
+    const int ray = ray_of(A, static_cast<int>(blockIdx.x) / colgroups);
+    if (ray < 0) return;   // the whole block
+    const int j = static_cast<int>(blockIdx.x) % colgroups * COLS + col;
+    const bool ok = j < A.nf;
+    const int jj = ok ? j : A.nf - 1;
+    int base, nlr;
+    const bool valid = ray_span(A, ray, base, nlr);
+    const int S = valid ? min(A.nsteps[ray], nlr - 1) : -1;   // never read past the ray's ds row or table
+    const int n = max(S - 1, 0);
+    const double *h = A.hds + static_cast<size_t>(ray) * A.ld;
+    const size_t nf = A.nf;
+    const AT *al = static_cast<const AT *>(A.alpha) + static_cast<size_t>(base) * nf + jj;
+    const double *Tl = A.T + base;
+    const int run = (n + SEGS - 1) / SEGS;
+    const int p0 = 1 + min(seg * run, n), p1 = 1 + min((seg + 1) * run, n);   // points [p0, p1)
+    double tot = 0.0, before = 0.0;
+    bool bad = false;   // a NaN half step or temperature: no cut (path_has_nan)
+    if (p0 < p1) {
+        before = static_cast<double>(al[(p0 - 1) * nf]);
+        double a0 = before;
+#pragma unroll 4
+        for (int p = p0; p < p1; ++p) {
+            const double a1 = static_cast<double>(al[p * nf]);
+            tot = tot + (a0 + a1) * h[p - 1];
+            bad = bad || __builtin_isnan(h[p - 1]) || __builtin_isnan(Tl[p]);
+            a0 = a1;
+        }
+    }
+    // inclusive sums over the wavefront's runs of this column, then the wavefronts before it
+    double incl = tot;
+#pragma unroll
+    for (int o = COLS; o < kLanes; o <<= 1) {
+        const double v = __shfl_up(incl, o, kLanes);
+        if (lane >= o) incl = v + incl;
+    }
+    if (lane >= kLanes - COLS) part[0][wave][col] = incl;
+    bad = __syncthreads_or(bad);   // and orders etab and part
+    const double own = __shfl_up(incl, COLS, kLanes);   // (not incl - tot: tot may be infinite)
+    double tau = 0.0;
+    for (int w = 0; w < wave; ++w) tau += part[0][w][col];
+    if (lane >= COLS) tau += own;
+    const double cut = (A.tau_cut > 0.0 && !bad) ? A.tau_cut : 0.0;
+    double intW = 0.0, num = 0.0, a0 = before;
+    for (int p = p0; p < p1; ++p) {
+        if (cut > 0.0 && tau > cut) break;
+        const double a1 = static_cast<double>(al[p * nf]);
+        const double hb = h[p - 1];
+        tau = tau + (a0 + a1) * hb;
+        const double Wp = MODE == 1 ? 2.0 * a1 * expint_e2(tau) : a1 * exp_neg_tab(tau, etab);
+        const double hw = Wp * (hb + (p < n ? h[p] : 0.0));
+        intW = intW + hw;
+        num = num + Tl[p] * hw;
+        a0 = a1;
+    }
+#pragma unroll
+    for (int o = COLS; o < kLanes; o <<= 1) {
+        intW += __shfl_xor(intW, o, kLanes);
+        num += __shfl_xor(num, o, kLanes);
+    }
+    __syncthreads();   // part[0] has been read
+    if (lane < COLS) {
+        part[0][wave][col] = intW;
+        part[1][wave][col] = num;
+    }
+    __syncthreads();
+    if (threadIdx.x >= COLS || !ok) return;
+    intW = num = 0.0;
+    for (int w = 0; w < W; ++w) {
+        intW += part[0][w][col];
+        num += part[1][w][col];
+    }
+    const size_t o = static_cast<size_t>(ray) * A.nf + (A.cols ? A.cols[j] : j);
+    double Tb;
+    if (!valid)
+        Tb = __builtin_nan("");
+    else if (S < 0 || num < kTcmb)
+        Tb = kTcmb;
+    else
+        Tb = num / intW;
+    A.Tb[o] = Tb;
+    if (A.intW) A.intW[o] = (S < 0) ? 0.0 : intW;
+}
+
 // The forward sums of one ray (brightness.py:93-101) for the Jacobian and the adjoint:
 // the integrated weight D = intW, the T-weighted sum num and the last path point reached.
 // The optical-depth cut is checked after every 8 steps; the steps are taken 8 at a time,
@@ -1043,7 +1148,39 @@ __global__ __launch_bounds__(256) void table_cols_kernel(const T *in, int nl, in
 
 }  // namespace rbx
 
+// The steps are split over segments up to this many blocks of 16 columns: two blocks are resident
+// per CU, and past one round of them the walk's own wavefronts fill the latency.  Walk against
+// segments at 64 frequencies: point rays of 400 layers, FP64, 64 rays 42 -> 13 us, 128 rays 42 -> 19,
+// 256 rays 42 -> 35, 512 rays 43 -> 67 (FP32 22 -> 13, 22 -> 18, 23 -> 33); discs of 400 layers, 128 rays
+// 1033 -> 196 us, 256 rays 996 -> 379, 1024 rays 1044 -> 1498 (an E2 takes both forms most of their time).
+constexpr long long kSegPointBlocks = 512, kSegDiscBlocks = 2048;
+// Fewer blocks of 16 columns than this: blocks of 4 columns, four times the runs.
+constexpr long long kNarrowBlocks = 128;
+
+static int launch_integrate_segments(const rbx::IntArgs &A, hipStream_t st) {
+    const long long g16 = (A.nf + 15) / 16, g4 = (A.nf + 3) / 4;
+    const bool narrow = A.nray * g16 < kNarrowBlocks;
+    const int groups = static_cast<int>(narrow ? g4 : g16);
+    const dim3 grid(static_cast<unsigned>(static_cast<long long>(A.nray) * groups)), block(rbx::kSegThreads);
+#define RBX_SEG_LAUNCH(AT, MODE)                                                                                 \
+    do {                                                                                                         \
+        if (narrow) hipLaunchKernelGGL((rbx::integrate_segments_kernel<AT, MODE, 4>), grid, block, 0, st, A, groups); \
+        else hipLaunchKernelGGL((rbx::integrate_segments_kernel<AT, MODE, 16>), grid, block, 0, st, A, groups);  \
+    } while (0)
+    if (A.mode == 1) {
+        if (A.f32) RBX_SEG_LAUNCH(float, 1); else RBX_SEG_LAUNCH(double, 1);
+    } else {
+        if (A.f32) RBX_SEG_LAUNCH(float, 0); else RBX_SEG_LAUNCH(double, 0);
+    }
+#undef RBX_SEG_LAUNCH
+    return rbx::launch_status("integrate_segments_kernel");
+}
+
 static int launch_integrate(rbx::IntArgs A, const rbx_launch &L, void *stream) {
+    // a launch shape that names the walk's unroll or block order keeps the walk
+    const long long blocks16 = static_cast<long long>(A.nray) * ((A.nf + 15) / 16);
+    if (!L.int_unroll && !L.int_map && blocks16 <= (A.mode == 1 ? kSegDiscBlocks : kSegPointBlocks))
+        return launch_integrate_segments(A, static_cast<hipStream_t>(stream));
     const long long rblocks = (A.nray + rbx::kWaves - 1) / rbx::kWaves;
     // ray major pads the ray blocks to a multiple of the XCD count (padding blocks find no ray).
     // Built-in choice: ray major while the whole table fits one XCD's L2 (4 MiB) beside the
