@@ -556,32 +556,112 @@ __global__ __launch_bounds__(kThreads, 3) void alpha_far_kernel(AlphaArgs args) 
 }
 
 // ---- pass 2: near lines summed per tile, plus the series ----
+//
+// A near line is summed term by term only at the columns it is close to.  A term is analytic in
+// f but for its poles +-sqrt(p), so over an interval of columns [lo, hi] that lies well away from
+// them it is its Chebyshev interpolant on n nodes to rho^-n, rho the Bernstein ellipse (foci lo
+// and hi) through the nearest pole: n values stand for all the interval's columns.  Lines outside
+// rho = 3.2 are taken at nodes: 16 in FP32 mode (8e-9 of the line's value, below an FP32 term's
+// roundings), 32 in FP64 mode (7e-17; 16 nodes outside rho = 6, 4e-13, took the same time and left
+// tables 1e-13 to 3e-13 from 64 bits where the direct sums leave 1e-15).
+//
+// The tile's columns form a binary tree of intervals (whole tile, halves, ... down to leaves of 32
+// columns, 64 in FP64 mode).  A batch of 64 listed lines (neighbours in frequency, so they mostly
+// agree) takes the largest intervals that all of its lines are outside the ellipse of, at their
+// nodes, and a leaf that some line is close to at its columns.  Lanes are the points of one interval
+// times groups of lines: 4 groups at 16 nodes, 2 at 32 points.  The sums stay per interval until the
+// slot's last line; then their Chebyshev coefficients are formed and each column adds its ancestors'
+// series.  By points, 128-column tiles of 1024 columns over 0.3-300 GHz need about 95 (FP32) where
+// every column of every listed line was 250 per line and unit of ln f; what remains is half the
+// direct points' FP64 detunings and half deriving the listed lines and finding their intervals.
+// The pass, before -> now: 400 layers x 512 columns x 11000 lines 331 -> 208 us (FP32), 812 -> 332
+// (FP64); 800 x 1024 x 25553 1517 -> 1067, 4195 -> 1936; 600 x 1000 x 11000 FP64 1569 -> 725; 300 x 201
+// FP64 421 -> 231.  Four wavefronts per SIMD (about 100 B of scratch a lane) against three without:
+// 800 x 1024 1575 against 1771 us for the whole table (FP32), five 1502 but 256-column tiles slower.
+constexpr double kNodeRho = 3.2;
 
-// one wavefront's staged batch of kWaveBatch near lines (the layout sum_staged_f32 reads)
-constexpr int kWaveBatch = 64;
-struct WaveStage {
-    alignas(16) double D[2][kWaveBatch];
-    alignas(16) double h[2][kWaveBatch];
-    alignas(16) float2 ac[2][kWaveBatch];
-    alignas(16) float2 dh[2][kWaveBatch];
-    unsigned int fast[2][kThreads / 64];
+template <int K, bool F32>
+struct NearTree {
+    static constexpr int nodes = F32 ? 16 : 32;
+    static constexpr int width = F32 ? 32 : 64;         // columns of a leaf
+    static constexpr int leaves = 64 * K / width;
+    static constexpr int intervals = 2 * leaves;        // heap order: 1 the tile, 2i and 2i + 1 its halves
+    static constexpr int node_groups = 64 / nodes, col_groups = 64 / width;   // line groups
 };
 
-// FP64 mode: the (D, a, c, g, G) the direct FP64 sums read (sum_staged_f64)
+// cos(j pi / 64), j = 0..127
+constexpr int kCosTab = 128;
+__constant__ double kCos64[kCosTab] = {
+    1.0, 0.9987954562051724, 0.9951847266721969, 0.989176509964781,
+    0.9807852804032304, 0.970031253194544, 0.9569403357322088, 0.9415440651830208,
+    0.9238795325112867, 0.9039892931234433, 0.881921264348355, 0.8577286100002721,
+    0.8314696123025452, 0.8032075314806449, 0.773010453362737, 0.7409511253549591,
+    0.7071067811865476, 0.6715589548470184, 0.6343932841636455, 0.5956993044924334,
+    0.5555702330196022, 0.5141027441932218, 0.47139673682599764, 0.4275550934302821,
+    0.3826834323650898, 0.33688985339222005, 0.2902846772544624, 0.2429801799032639,
+    0.19509032201612828, 0.14673047445536175, 0.0980171403295606, 0.049067674327418015,
+    0.0, -0.049067674327418015, -0.0980171403295606, -0.14673047445536175,
+    -0.19509032201612828, -0.2429801799032639, -0.2902846772544624, -0.33688985339222005,
+    -0.3826834323650898, -0.4275550934302821, -0.47139673682599764, -0.5141027441932218,
+    -0.5555702330196022, -0.5956993044924334, -0.6343932841636455, -0.6715589548470184,
+    -0.7071067811865476, -0.7409511253549591, -0.773010453362737, -0.8032075314806449,
+    -0.8314696123025452, -0.8577286100002721, -0.881921264348355, -0.9039892931234433,
+    -0.9238795325112867, -0.9415440651830208, -0.9569403357322088, -0.970031253194544,
+    -0.9807852804032304, -0.989176509964781, -0.9951847266721969, -0.9987954562051724,
+    -1.0, -0.9987954562051724, -0.9951847266721969, -0.989176509964781,
+    -0.9807852804032304, -0.970031253194544, -0.9569403357322088, -0.9415440651830208,
+    -0.9238795325112867, -0.9039892931234433, -0.881921264348355, -0.8577286100002721,
+    -0.8314696123025452, -0.8032075314806449, -0.773010453362737, -0.7409511253549591,
+    -0.7071067811865476, -0.6715589548470184, -0.6343932841636455, -0.5956993044924334,
+    -0.5555702330196022, -0.5141027441932218, -0.47139673682599764, -0.4275550934302821,
+    -0.3826834323650898, -0.33688985339222005, -0.2902846772544624, -0.2429801799032639,
+    -0.19509032201612828, -0.14673047445536175, -0.0980171403295606, -0.049067674327418015,
+    0.0, 0.049067674327418015, 0.0980171403295606, 0.14673047445536175,
+    0.19509032201612828, 0.2429801799032639, 0.2902846772544624, 0.33688985339222005,
+    0.3826834323650898, 0.4275550934302821, 0.47139673682599764, 0.5141027441932218,
+    0.5555702330196022, 0.5956993044924334, 0.6343932841636455, 0.6715589548470184,
+    0.7071067811865476, 0.7409511253549591, 0.773010453362737, 0.8032075314806449,
+    0.8314696123025452, 0.8577286100002721, 0.881921264348355, 0.9039892931234433,
+    0.9238795325112867, 0.9415440651830208, 0.9569403357322088, 0.970031253194544,
+    0.9807852804032304, 0.989176509964781, 0.9951847266721969, 0.9987954562051724,
+};
+
+// one wavefront's staged batch of kWaveBatch near lines
+constexpr int kWaveBatch = 64;
+struct WaveStage {
+    alignas(16) double D[kWaveBatch];    // Ds
+    alignas(16) double h[kWaveBatch];
+    alignas(16) float2 ac[kWaveBatch];   // a, c (scaled)
+    alignas(16) float2 dh[kWaveBatch];   // Ds less the interval's x centre, and h, rounded to FP32
+};
+
+// FP64 mode: the (D, a, c, g, G) of the direct FP64 sums
 struct WaveStage64 {
-    double D[2][kWaveBatch], a[2][kWaveBatch], c[2][kWaveBatch], g[2][kWaveBatch], G[2][kWaveBatch];
+    alignas(16) double D[kWaveBatch], a[kWaveBatch], c[kWaveBatch], g[kWaveBatch], G[kWaveBatch];
+};
+
+// An interval of the tile's columns in f, of one range (kFarRanges); hi < lo: no columns
+struct NearInterval {
+    double c, r;          // centre, half width
+    float lo, hi, thr;    // thr: the least |z - lo| + |z - hi| of a pole outside the ellipse
 };
 
 template <int K, bool F32>
 struct NearShared {
+    using Tree = NearTree<K, F32>;
     std::conditional_t<F32, WaveStage, WaveStage64> st[kThreads / 64];
+    // the wavefronts' sums at the intervals' nodes and at the columns
+    double node[kThreads / 64][Tree::intervals][Tree::nodes];
+    double column[kThreads / 64][64 * K];
     union {
         unsigned short list[kListWords * 32];   // a window's near lines
-        double red[kThreads / 64][K][64];       // the wavefronts' partial sums at a slot's end
+        double cheb[2][Tree::intervals][Tree::nodes];   // node sums, Chebyshev coefficients
     };
     double far[kFarMom];
-    WaveRanges rng;
+    NearInterval iv[kFarRanges][Tree::intervals];
+    double cosines[kCosTab];
     int wsum[kThreads / 64];
+    int used;                        // some wavefront has added to node or column
     alignas(16) double prep[2][8];   // the segment's coefficient sets (read from LDS while deriving)
     double scale[2];                 // and their FP32 weight scales
 };
@@ -639,18 +719,159 @@ __device__ __forceinline__ void derive_near(int seg, int v, const DevBlock &B, i
     }
 }
 
+// v summed over the wavefront's `G` line groups (lane bits 5, then 4), in every lane
+template <int G>
+__device__ __forceinline__ double group_sum(double v) {
+    using Words = unsigned int __attribute__((ext_vector_type(2)));
+    auto add = [](double y, auto &&swap) {
+        const Words w = __builtin_bit_cast(Words, y);
+        const auto lo = swap(w.x), hi = swap(w.y);
+        return __builtin_bit_cast(double, Words{lo[0], hi[0]}) + __builtin_bit_cast(double, Words{lo[1], hi[1]});
+    };
+    if constexpr (G >= 4) v = add(v, [](unsigned int q) { return __builtin_amdgcn_permlane16_swap(q, q, false, false); });
+    if constexpr (G >= 2) v = add(v, [](unsigned int q) { return __builtin_amdgcn_permlane32_swap(q, q, false, false); });
+    return v;
+}
+
+// The pole in f nearest the positive axis of (x - Ds)^2 + h: sqrt(Ds + i sqrt(h)) for a complex
+// pair; for h < 0 (a coupling or width beyond the centre: both poles real and negative) i times the
+// root of the smaller modulus.  Anything else gives NaN, which is close to every interval.
+__device__ __forceinline__ float2 pole_in_f(double Ds, double h) {
+    const float d = static_cast<float>(Ds), q = __builtin_amdgcn_sqrtf(fabsf(static_cast<float>(h)));
+    if (h >= 0.0) {
+        const float m = __builtin_amdgcn_sqrtf(static_cast<float>(fma(Ds, Ds, h)));
+        const float big = __builtin_amdgcn_sqrtf(0.5f * (m + fabsf(d)));
+        const float small = 0.5f * q / big;
+        return d >= 0.0f ? make_float2(big, small) : make_float2(small, big);
+    }
+    return make_float2(0.0f, d < 0.0f && q <= -d ? __builtin_amdgcn_sqrtf(-d - q) : NAN);
+}
+
+__device__ __forceinline__ bool outside(const float2 &z, const NearInterval &I) {
+    const float a = z.x - I.lo, b = z.x - I.hi, y2 = z.y * z.y;
+    return __builtin_amdgcn_sqrtf(fmaf(a, a, y2)) + __builtin_amdgcn_sqrtf(fmaf(b, b, y2)) >= I.thr;
+}
+
+// Sum of the staged lines' terms at this lane's point x, over the pairs of lines g, g + G, ... of
+// the batch's first `npairs` (a multiple of 4 G), two lines over one denominator and blocks of 8
+// lines in FP32.  `fast`: bit j = lines [8 j, 8 j + 8) take the all-FP32 denominator
+// (dx - dD)^2 + h, dx and dD the distances of x and Ds from the interval's centre; the others form
+// it in FP64 (as sum_staged_f32).
+template <int G>
+__device__ __forceinline__ double sum_pairs(const WaveStage &st, int g, int npairs, double x, float dx,
+                                            unsigned int fast) {
+    const float xf = static_cast<float>(x);
+    constexpr unsigned int kAll = (1u << G) - 1u;
+    double acc = 0.0;
+    for (int p0 = 0; p0 < npairs; p0 += 4 * G) {
+        float p = 0.0f;
+        if (((fast >> (p0 / 4)) & kAll) == kAll) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const float4 dp = reinterpret_cast<const float4 *>(st.dh)[p0 + u * G + g];
+                const float4 qp = reinterpret_cast<const float4 *>(st.ac)[p0 + u * G + g];
+                const float d1 = dx - dp.x, d2 = dx - dp.z;
+                const float e1 = fmaf(d1, d1, dp.y), e2 = fmaf(d2, d2, dp.w);
+                const float n1 = fmaf(qp.x, xf, qp.y), n2 = fmaf(qp.z, xf, qp.w);
+                p = fmaf(fmaf(n2, e1, n1 * e2), __builtin_amdgcn_rcpf(e1 * e2), p);
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const double2 Dp = reinterpret_cast<const double2 *>(st.D)[p0 + u * G + g];
+                const double2 hp = reinterpret_cast<const double2 *>(st.h)[p0 + u * G + g];
+                const float4 qp = reinterpret_cast<const float4 *>(st.ac)[p0 + u * G + g];
+                const double d1 = x - Dp.x, d2 = x - Dp.y;
+                const float e1 = static_cast<float>(fma(d1, d1, hp.x)), e2 = static_cast<float>(fma(d2, d2, hp.y));
+                const float n1 = fmaf(qp.x, xf, qp.y), n2 = fmaf(qp.z, xf, qp.w);
+                p = fmaf(fmaf(n2, e1, n1 * e2), __builtin_amdgcn_rcpf(e1 * e2), p);
+            }
+        }
+        acc += static_cast<double>(p);
+    }
+    return acc;
+}
+
+// the same in FP64 (the terms of sum_staged_f64)
+template <int G>
+__device__ __forceinline__ double sum_pairs(const WaveStage64 &st, int g, int npairs, double x, float, unsigned int) {
+    double acc = 0.0;
+#pragma unroll 2
+    for (int p = g; p < npairs; p += G) {
+        const double2 D = reinterpret_cast<const double2 *>(st.D)[p], a = reinterpret_cast<const double2 *>(st.a)[p];
+        const double2 c = reinterpret_cast<const double2 *>(st.c)[p], gg = reinterpret_cast<const double2 *>(st.g)[p];
+        const double2 GG = reinterpret_cast<const double2 *>(st.G)[p];
+        const double d1 = x - D.x, d2 = x - D.y;
+        const double n1 = fma(a.x, x, c.x), n2 = fma(a.y, x, c.y);
+        const double e1 = fma(d1, d1, fma(gg.x, x, GG.x)), e2 = fma(d2, d2, fma(gg.y, x, GG.y));
+        acc += fma(n1, e2, n2 * e1) * recip(e1 * e2);
+    }
+    return acc;
+}
+
+// A batch's staged lines added at the tree's points: this lane's line has shifted centre Ds, h and
+// pole z (`line` false: padding, a zero term); columns' x of the leaves from `colx`.
+template <int K, bool F32, class ColX>
+__device__ __forceinline__ void sum_tree(NearShared<K, F32> &sh, int rv, bool line, double Ds, double h, int count,
+                                         double inv_scale, const ColX &colx) {
+    using Tree = NearTree<K, F32>;
+    const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    auto &st = sh.st[wave];
+    const float2 z = pole_in_f(Ds, h);
+    const double node = sh.cosines[(2 * (lane % Tree::nodes) + 1) * (kCosTab / 4 / Tree::nodes)];
+    unsigned int pending = 2u;
+#pragma unroll 1
+    for (int i = 1; i < Tree::intervals; ++i) {
+        if (!((pending >> i) & 1u)) continue;
+        const NearInterval I = sh.iv[rv][i];
+        if (!(I.lo <= I.hi)) continue;   // no columns
+        const bool nodes = __all(!line || outside(z, I));
+        if (!nodes && i < Tree::leaves) {
+            pending |= 3u << (2 * i);
+            continue;
+        }
+        const double xc = I.c * I.c;
+        unsigned int fast = 0u;
+        if constexpr (F32) {
+            // FP32 denominators: the distances' roundings stay within a few of x - Ds (or of the
+            // root of h beside it) past twice the interval's half width in x, as they do for every
+            // line outside the ellipse; h < 0 must not cancel (x - Ds)^2
+            const double dD = Ds - xc, lo2 = static_cast<double>(I.lo) * I.lo - Ds;
+            const float rx = static_cast<float>(I.r * (2.0 * I.c + I.r)), dDf = static_cast<float>(dD);
+            const bool ok = h >= 0.0 ? (nodes || fabsf(dDf) >= 2.0f * rx || static_cast<float>(h) >= rx * rx)
+                                     : (lo2 > 0.0 && lo2 * lo2 >= -4.0 * h && (nodes || fabsf(dDf) >= 2.0f * rx));
+            fast = full_chunks(__ballot(!line || ok));
+            wave_sync();   // (the interval before has been summed)
+            st.dh[lane] = make_float2(dDf, static_cast<float>(h));
+            wave_sync();
+        }
+        if (nodes) {
+            constexpr int G = Tree::node_groups;
+            const double f = fma(I.r, node, I.c), x = f * f;
+            const double s = group_sum<G>(sum_pairs<G>(st, lane / Tree::nodes, (count + 8 * G - 1) / (8 * G) * (4 * G), x,
+                                                       static_cast<float>(x - xc), fast));
+            double &v = sh.node[wave][i][lane % Tree::nodes];
+            if (lane < Tree::nodes) v = fma(s, inv_scale, v);
+        } else {
+            constexpr int G = Tree::col_groups;
+            const int k = (i - Tree::leaves) * Tree::width + lane % Tree::width;
+            const double x = colx(k);
+            const double s = group_sum<G>(sum_pairs<G>(st, lane / Tree::width, (count + 8 * G - 1) / (8 * G) * (4 * G), x,
+                                                       static_cast<float>(x - xc), fast));
+            double &v = sh.column[wave][k];
+            if (lane < Tree::width) v = fma(s, inv_scale, v);
+        }
+    }
+}
+
 // near lines of one segment and coefficient set v, listed from the tile's mask words; each
-// wavefront sums its own batches of kWaveBatch listed lines (batches w, w + 4, ...), staged
-// in its own LDS and fetched one batch ahead into registers.  `so` = the stream's first line
-// in the staged-line arrays.
-template <int K, bool F32, class Derive>
-__device__ void near_sum(const AlphaArgs &A, int n, const Derive &derive, int v, bool mixed, bool uni,
-                         const unsigned int *mask,
-                         int nwords, int var, const int (&set)[K], const double (&x)[K], const float (&xf)[K],
-                         double (&acc)[K], NearShared<K, F32> &sh) {
+// wavefront sums its own batches of kWaveBatch listed lines (batches w, w + 4, ...), staged in its
+// own LDS.
+template <int K, bool F32, class Derive, class ColX>
+__device__ void near_sum(int n, const Derive &derive, int rv, const unsigned int *mask, int nwords, double inv_scale,
+                         const ColX &colx, NearShared<K, F32> &sh) {
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
     auto &st = sh.st[wave];
-    const double lo = sh.rng.lo[var][0], hi = sh.rng.hi[var][0];
     for (int w0 = 0; w0 < nwords; w0 += kListWords) {
         const int wi = w0 + tid;
         const unsigned int bits = (tid < kListWords && wi < nwords) ? mask[wi] : 0u;
@@ -671,69 +892,95 @@ __device__ void near_sum(const AlphaArgs &A, int n, const Derive &derive, int v,
         }
         for (unsigned int b = bits; b != 0u; b &= b - 1u)
             sh.list[pos++] = static_cast<unsigned short>(tid * 32 + __builtin_ctz(b));
+        if (total > 0 && tid == 0) sh.used = 1;
         __syncthreads();
         // listed line e's coefficients, derived from its catalogue row when its batch is
         // staged (past the list: a zero term): FP32 (Ds, h, a s, c s), FP64 (D, a, c, g, G)
         const int nb = (total + kWaveBatch - 1) / kWaveBatch;
         for (int b = wave; b < nb; b += kThreads / 64) {
-            const int cntp = (min(kWaveBatch, total - b * kWaveBatch) + kSub - 1) / kSub * kSub;
             const int e = b * kWaveBatch + lane;
             const int i = e < total ? w0 * 32 + sh.list[e] : n;
             double c5[5] = {0.0, F32 ? 1.0 : 0.0, 0.0, 0.0, 1.0};
             float2 ac = make_float2(0.0f, 0.0f);
             if (i < n) derive(i, c5, ac);
+            double Ds = c5[0], h = c5[1];
+            wave_sync();   // (the batch before has been summed)
             if constexpr (F32) {
-                st.D[v][lane] = c5[0];
-                st.h[v][lane] = c5[1];
-                st.ac[v][lane] = ac;
-                st.dh[v][lane] = make_float2(static_cast<float>(c5[0]), static_cast<float>(c5[1]));
-                if (mixed) {   // the other set's columns add nothing
-                    st.D[1 - v][lane] = 0.0;
-                    st.h[1 - v][lane] = 1.0;
-                    st.ac[1 - v][lane] = make_float2(0.0f, 0.0f);
-                    st.dh[1 - v][lane] = make_float2(0.0f, 1.0f);
-                }
-                const unsigned int fb = full_chunks(__ballot(fp32_safe(c5[0], c5[1], lo, hi)));
-                if (lane == 0) st.fast[v][wave] = fb;
+                st.D[lane] = Ds;
+                st.h[lane] = h;
+                st.ac[lane] = ac;
             } else {
-                st.D[v][lane] = c5[0];
-                st.a[v][lane] = c5[1];
-                st.c[v][lane] = c5[2];
-                st.g[v][lane] = c5[3];
-                st.G[v][lane] = c5[4];
-                if (mixed) {
-                    st.D[1 - v][lane] = 0.0;
-                    st.a[1 - v][lane] = 0.0;
-                    st.c[1 - v][lane] = 0.0;
-                    st.g[1 - v][lane] = 0.0;
-                    st.G[1 - v][lane] = 1.0;
-                }
+                st.D[lane] = c5[0];
+                st.a[lane] = c5[1];
+                st.c[lane] = c5[2];
+                st.g[lane] = c5[3];
+                st.G[lane] = c5[4];
+                shifted_denominator(CoefT<double>{c5[0], c5[1], c5[2], c5[3], c5[4]}, Ds, h);
             }
             wave_sync();
-            if constexpr (F32) {
-                if (uni)
-                    sum_staged_f32<K, true>(st, set, 0, cntp, x, xf, acc);
-                else
-                    sum_staged_f32<K, false>(st, set, 0, cntp, x, xf, acc);
-            } else {
-                if (uni)
-                    sum_staged_f64<K, true>(st, set, 0, cntp, x, acc);
-                else
-                    sum_staged_f64<K, false>(st, set, 0, cntp, x, acc);
-            }
-            wave_sync();
+            sum_tree<K, F32>(sh, rv, i < n, Ds, h, min(kWaveBatch, total - b * kWaveBatch), inv_scale, colx);
         }
         __syncthreads();   // every wavefront is done with this window's list
     }
 }
 
+// The sums at the tree's points brought to column `tid` (threads below the tile's width): the
+// wavefronts' and line groups' sums in order, the intervals' Chebyshev coefficients, and the series
+// of the column's ancestors at its f.  Clears the sums; called by the whole block.
 template <int K, bool F32>
-__global__ __launch_bounds__(kThreads, K >= 4 ? 2 : 4) void alpha_near_kernel(AlphaArgs args) {
+__device__ double tree_to_column(NearShared<K, F32> &sh, int rv, double f) {
+    using Tree = NearTree<K, F32>;
+    const int tid = threadIdx.x;
+    __syncthreads();
+    if (!sh.used) return 0.0;   // (the same for every thread; nothing has been added)
+    const int i0 = tid / Tree::nodes, k0 = tid % Tree::nodes;
+    if (i0 >= 1 && i0 < Tree::intervals) {
+        double s = 0.0;
+        for (int w = 0; w < kThreads / 64; ++w) s += sh.node[w][i0][k0];
+        sh.cheb[0][i0][k0] = s;
+    }
+    __syncthreads();
+    if (i0 >= 1 && i0 < Tree::intervals) {
+        double s = 0.0;
+#pragma unroll
+        for (int k = 0; k < Tree::nodes; ++k)
+            s = fma(sh.cheb[0][i0][k], sh.cosines[(k0 * (2 * k + 1) * (kCosTab / 4 / Tree::nodes)) % kCosTab], s);
+        sh.cheb[1][i0][k0] = s * ((k0 == 0 ? 1.0 : 2.0) / Tree::nodes);
+    }
+    __syncthreads();
+    double out = 0.0;
+    if (tid < 64 * K) {
+        const int leaf = tid / Tree::width;
+        for (int w = 0; w < kThreads / 64; ++w) out += sh.column[w][tid];
+        for (int i = Tree::leaves + leaf; i >= 1; i >>= 1) {
+            const NearInterval &I = sh.iv[rv][i];
+            const double u = I.r > 0.0 ? (f - I.c) / I.r : 0.0, u2 = 2.0 * u;
+            double b1 = 0.0, b2 = 0.0;   // Clenshaw
+#pragma unroll
+            for (int m = Tree::nodes - 1; m >= 1; --m) {
+                const double b0 = fma(u2, b1, sh.cheb[1][i][m] - b2);
+                b2 = b1;
+                b1 = b0;
+            }
+            out += fma(u, b1, sh.cheb[1][i][0] - b2);
+        }
+    }
+    __syncthreads();
+    for (int e = tid; e < (kThreads / 64) * Tree::intervals * Tree::nodes; e += kThreads) (&sh.node[0][0][0])[e] = 0.0;
+    for (int e = tid; e < (kThreads / 64) * 64 * K; e += kThreads) (&sh.column[0][0])[e] = 0.0;
+    if (tid == 0) sh.used = 0;
+    __syncthreads();
+    return out;
+}
+
+template <int K, bool F32>
+__global__ __launch_bounds__(kThreads, 4) void alpha_near_kernel(AlphaArgs args) {
 #if defined(__HIP_DEVICE_COMPILE__)
     const AlphaArgs &A = *reinterpret_cast<const AlphaArgs *>(__builtin_amdgcn_kernarg_segment_ptr());
 #else
     const AlphaArgs &A = args;   // (host pass: never run)
 #endif
+    using Tree = NearTree<K, F32>;
     __shared__ NearShared<K, F32> sh;
     // layer fastest: blocks are dealt to the XCDs in turn, so each XCD gets every tile (the
     // tiles' near fractions differ several-fold) rather than one tile of every layer.  Last
@@ -747,37 +994,57 @@ __global__ __launch_bounds__(kThreads, K >= 4 ? 2 : 4) void alpha_near_kernel(Al
     int c0, c1;
     tile_cols(A, tile, c0, c1);
     const int tsets = tile_sets(A, c0, c1);
-    const bool mixed = tsets == 3;
+    const bool mixed = tsets == 3;   // the tile straddles the switch between the inversion sets
 
-    int col[K], set[K];
-    bool ok[K];
-    double x[K], xn[K];
-    float xf[K], xnf[K];
+    // thread tid owns column c0 + tid
+    const int col = c0 + tid;
+    const bool ok = tid < 64 * K && col < A.nf;
+    const int cc = min(col, A.nf - 1);
+    const int set = cc < A.nf_low ? 0 : 1;
+    const double f = A.freq[cc], fn = A.freq_nh3 ? A.freq_nh3[cc] : f;
+
+    // the tree's intervals: wavefront v the range v, leaves first (LDS: lo and hi in c and r)
+    static_assert(kFarRanges == kThreads / 64, "a wavefront per range");
 #pragma unroll
     for (int k = 0; k < K; ++k) {
-        col[k] = c0 + lane + k * 64;
-        ok[k] = col[k] < A.nf;
-        const int cc = min(col[k], A.nf - 1);
-        set[k] = cc < A.nf_low ? 0 : 1;
-        const double f = A.freq[cc];
-        const double fn = A.freq_nh3 ? A.freq_nh3[cc] : f;
-        x[k] = f * f;
-        xn[k] = fn * fn;
-        xf[k] = static_cast<float>(x[k]);
-        xnf[k] = static_cast<float>(xn[k]);
-    }
-    const bool uni_set = !mixed;   // every column of the tile reads one inversion set
-
-    if (wave == 0) {
-        double lo[kFarRanges], hi[kFarRanges];
-        tile_ranges(A, tile, lo, hi);
-        if (lane < kThreads / 64) {
+        const int cl = c0 + k * 64 + lane;
+        const bool in = cl < c1 && (wave < 2 || (cl < A.nf_low ? 2 : 3) == wave);
+        const int ccl = min(cl, A.nf - 1);
+        const double fl = wave > 0 && A.freq_nh3 ? A.freq_nh3[ccl] : A.freq[ccl];
+        double lo = in ? fl : INFINITY, hi = in ? fl : -INFINITY;
 #pragma unroll
-            for (int v = 0; v < 2; ++v) {
-                sh.rng.lo[v][lane] = lo[v];
-                sh.rng.hi[v][lane] = hi[v];
-            }
+        for (int m = Tree::width / 2; m > 0; m >>= 1) {
+            lo = fmin(lo, __shfl_xor(lo, m));
+            hi = fmax(hi, __shfl_xor(hi, m));
         }
+        if (lane % Tree::width == 0) {
+            NearInterval &I = sh.iv[wave][Tree::leaves + k * Tree::col_groups + lane / Tree::width];
+            I.c = lo;
+            I.r = hi;
+        }
+    }
+    wave_sync();
+#pragma unroll
+    for (int lev = Tree::leaves / 2; lev >= 1; lev /= 2) {
+        if (lane >= lev && lane < 2 * lev) {
+            const NearInterval a = sh.iv[wave][2 * lane], b = sh.iv[wave][2 * lane + 1];
+            sh.iv[wave][lane].c = fmin(a.c, b.c);
+            sh.iv[wave][lane].r = fmax(a.r, b.r);
+        }
+        wave_sync();
+    }
+    if (lane >= 1 && lane < Tree::intervals) {
+        NearInterval &I = sh.iv[wave][lane];
+        const double lo = I.c, hi = I.r;
+        I.lo = static_cast<float>(lo);
+        I.hi = static_cast<float>(hi);
+        I.c = 0.5 * (lo + hi);
+        I.r = 0.5 * (hi - lo);
+        // The margin covers the FP32 roundings of lo, hi and the poles; f < 0: never outside.  A
+        // node's f is rounded to 2^-53 c, which moves a term by up to about 2^-53 c / r of itself:
+        // FP64 mode takes no nodes in narrow intervals.
+        const bool use = lo >= 0.0 && (F32 || 64.0 * I.r >= I.c);
+        I.thr = use ? static_cast<float>(I.r * (kNodeRho + 1.0 / kNodeRho) + 1.0e-6 * hi) : INFINITY;
     }
     for (int e = tid; e < kFarMom; e += kThreads) {
         double s = 0.0;
@@ -785,6 +1052,10 @@ __global__ __launch_bounds__(kThreads, K >= 4 ? 2 : 4) void alpha_near_kernel(Al
             s += A.far_mom[((static_cast<size_t>(layer) * nsplit + p) * A.tiles_total + tile) * kFarMom + e];
         sh.far[e] = s;
     }
+    if (tid < kCosTab) sh.cosines[tid] = kCos64[tid];
+    for (int e = tid; e < (kThreads / 64) * Tree::intervals * Tree::nodes; e += kThreads) (&sh.node[0][0][0])[e] = 0.0;
+    for (int e = tid; e < (kThreads / 64) * 64 * K; e += kThreads) (&sh.column[0][0])[e] = 0.0;
+    if (tid == 0) sh.used = 0;
     if (tile == 0 && tid == 0) {
         double b = 0.0;
         for (int p = 0; p < nsplit; ++p) b += A.far_base[static_cast<size_t>(p) * A.nl + layer];
@@ -796,39 +1067,25 @@ __global__ __launch_bounds__(kThreads, K >= 4 ? 2 : 4) void alpha_near_kernel(Al
     const int touched = plan.slots(0, 1);
     const size_t plane = static_cast<size_t>(A.nl) * A.nf;
     const unsigned int *masks = A.near + (static_cast<size_t>(layer) * A.tiles_total + tile) * A.far_words;
-    double acc[K] = {};
-    auto series = [&](int q, int k) {
+    auto series = [&](int q) {
+        const double x = f * f, xn = fn * fn;
         switch (q) {
-            case kSlotH2o: return far_eval(sh.far + 0 * 2 * kFarTerms, x[k]);
-            case kSlotH2s: return far_eval(sh.far + 1 * 2 * kFarTerms, x[k]);
+            case kSlotH2o: return far_eval(sh.far + 0 * 2 * kFarTerms, x);
+            case kSlotH2s: return far_eval(sh.far + 1 * 2 * kFarTerms, x);
             case kSlotNh3:
-                return far_eval(sh.far + (2 + set[k]) * 2 * kFarTerms, xn[k]) +
-                       far_eval(sh.far + 4 * 2 * kFarTerms, xn[k]);
-            default: return far_eval(sh.far + 5 * 2 * kFarTerms, x[k]);
+                return far_eval(sh.far + (2 + set) * 2 * kFarTerms, xn) + far_eval(sh.far + 4 * 2 * kFarTerms, xn);
+            default: return far_eval(sh.far + 5 * 2 * kFarTerms, x);
         }
     };
-    // the wavefronts' partial sums of the same columns, added in wavefront order, plus the series
+    double acc = 0.0;   // column tid's sum of the current slot
     auto store = [&](int q) {
-        if (touched & (1 << q)) {
-#pragma unroll
-            for (int k = 0; k < K; ++k) sh.red[wave][k][lane] = acc[k];
-            __syncthreads();
-            if (wave == 0) {
-                double *w = A.ws + static_cast<size_t>(q) * plane + static_cast<size_t>(layer) * A.nf;
-#pragma unroll
-                for (int k = 0; k < K; ++k) {
-                    double t = sh.red[0][k][lane];
-#pragma unroll
-                    for (int ww = 1; ww < kThreads / 64; ++ww) t += sh.red[ww][k][lane];
-                    if (ok[k]) w[col[k]] = t + series(q, k);
-                }
-            }
-            __syncthreads();
-        }
-#pragma unroll
-        for (int k = 0; k < K; ++k) acc[k] = 0.0;
+        if ((touched & (1 << q)) && ok)
+            A.ws[static_cast<size_t>(q) * plane + static_cast<size_t>(layer) * A.nf + col] = acc + series(q);
+        acc = 0.0;
     };
     for (int seg = 0; seg < kSegs; ++seg) {
+        const bool inv = seg == 2;
+        const int var = kSegVar[seg];
         if (plan.nr[seg] > 0) {
             // the segment's coefficient sets and weight scales go to LDS and are read there
             // while deriving (held in registers across the line sums they would crowd out the
@@ -842,40 +1099,31 @@ __global__ __launch_bounds__(kThreads, K >= 4 ? 2 : 4) void alpha_near_kernel(Al
                     sh.scale[tid - 16] = w;
             }
             __syncthreads();
-            const bool inv = seg == 2;
-            const int var = kSegVar[seg];
             const DevBlock &B = A.cat.blk[kSegKind[seg]];
             const int nwords = plan.nr[seg] * (kThreads / 32);
-            double a2[K] = {}, xv[K];
-            float xfv[K];
-            int sets[K];
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                xv[k] = var ? xn[k] : x[k];
-                xfv[k] = var ? xnf[k] : xf[k];
-                sets[k] = inv ? set[k] : 0;
-            }
+            auto colx = [&](int k) {
+                const int ck = min(c0 + k, A.nf - 1);
+                const double fk = var && A.freq_nh3 ? A.freq_nh3[ck] : A.freq[ck];
+                return fk * fk;
+            };
 #pragma unroll 1
             for (int v = 0; v < 2; ++v) {
                 if (inv ? !((tsets >> v) & 1) : v > 0) continue;
                 const unsigned int *mk = masks + A.far_off[kSegStream[seg] + (inv ? v : 0)];
                 const double sv = sh.scale[v];
                 auto derive = [&](int i, double (&c5)[5], float2 &ac) { derive_near<F32>(seg, v, B, i, sh.prep, sv, c5, ac); };
-                near_sum<K, F32>(A, B.n, derive, inv ? v : 0, inv && mixed, inv ? uni_set : true, mk, nwords, var, sets,
-                                 xv, xfv, a2, sh);
-            }
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                const double sc = sh.scale[inv ? set[k] : 0];
-                if (seg == 0 || seg == 1 || seg == 5)
-                    acc[k] = a2[k] / sc;
-                else
-                    acc[k] += a2[k] / sc;
+                const int rv = inv ? 2 + v : var;
+                near_sum<K, F32>(B.n, derive, rv, mk, nwords, 1.0 / sv, colx, sh);   // (sv is a power of two)
+                // of a tile of both sets only set v's columns, over their own intervals
+                if (inv && mixed) {
+                    const double s = tree_to_column<K, F32>(sh, rv, fn);
+                    if (set == v) acc += s;
+                }
             }
         }
-        if (seg == 0) store(kSlotH2o);
-        if (seg == 1) store(kSlotH2s);
-        if (seg == 4) store(kSlotNh3);
-        if (seg == 5) store(kSlotPh3);
+        if (seg == 0 || seg == 1 || seg == 4 || seg == 5) {
+            acc += tree_to_column<K, F32>(sh, var, var ? fn : f);
+            store(seg == 0 ? kSlotH2o : seg == 1 ? kSlotH2s : seg == 4 ? kSlotNh3 : kSlotPh3);
+        }
     }
 }
