@@ -164,13 +164,15 @@ int rbx_device_count(int *count);
  * launch, ...) on any thread. */
 typedef struct rbx_launch {
     int alpha_k;        /* frequencies per lane of the forward line sums: 1, 2 or 4 (built in:
-                           2 from 256 frequencies up, else 1) */
+                           2 from 256 frequencies up, else 1; the series path 4 from 768 up with
+                           enough layers) */
     int alpha_series;   /* rbx_alpha: 1 sums every line at every frequency; 2 sums per wavefront
                            tile only the lines whose poles lie within a factor 3 (FP32) or 6.7
                            (FP64) of the tile's x = f^2 range and adds the others as 16-term power
                            series (at most 8e-7 / 8e-12 of a far line's value: FP32 tables within
                            3e-7 of FP64 as the direct sums, FP64 tables within 1e-11 of the direct
-                           FP64 sums); built in: 2 for requests of 4 or more wavefront tiles while
+                           FP64 sums); built in: 2 for requests of 4 or more wavefront tiles (fewer in
+                           FP64 past 128 frequencies, in FP32 past 256, when layers x lines are many) while
                            the workspace (the tiles' moments and near-line masks: about 0.1 MB per
                            layer at 1024 frequencies and 25553 lines) stays under 4 GiB, else 1 */
     int alpha_split;    /* parts each layer's direct line sums are split into: 1..16 (built in: a

@@ -1622,6 +1622,16 @@ static int alpha_tile_k(int nf, const rbx_launch &L) {
     return nf >= 256 ? 2 : 1;
 }
 
+// The series path's tiles: from 768 columns up 256 of them, where that leaves at least 1600 blocks (two
+// rounds of the resident ones): a near line is listed and derived for fewer tiles.  Whole tables, 128
+// against 256 columns: 600 layers x 1000 columns FP64 933 -> 830 us, 800 x 1024 1574 -> 1494 (FP32) and
+// 2290 -> 2167 us; 400 x 512, 800 blocks of 256 columns, 443 -> 451 and 559 -> 558.
+static int series_tile_k(const AlphaArgs &A, const rbx_launch &L) {
+    const int k = alpha_tile_k(A.nf, L);
+    const bool wide = A.nf >= 768 && static_cast<long long>(A.nl) * ((A.nf + 255) / 256) >= 1600;
+    return L.alpha_k == 0 && wide ? 4 : k;
+}
+
 static void set_wave_tiles(AlphaArgs &A, int K) {
     A.tile_width = 64 * K;   // one wavefront tile
     A.tiles_total = (A.nf + A.tile_width - 1) / A.tile_width;
@@ -1688,16 +1698,25 @@ static int alpha_split(const AlphaArgs &A, const rbx_launch &L, int K, int preci
     return RBX_OK;
 }
 
-// far-line series (far.hpp): launch.alpha_series 1 off, 2 on; built in on for
-// requests of at least kSeriesMinTiles wavefront tiles while the workspace stays under
-// kSeriesMaxWorkspace.  (With fewer tiles few (line, tile) pairs are far and the extra pass
-// costs more than it saves: one 20-frequency tile of 150 layers took 0.37 ms per step against
-// 0.21 ms with the direct sums.)
+// far-line series (far.hpp): launch.alpha_series 1 off, 2 on; built in while the workspace stays under
+// kSeriesMaxWorkspace for requests of at least kSeriesMinTiles tiles of the direct sums' width, and of
+// fewer where the direct sums are long enough that the two passes' launches (about 50 us) pay.  (One
+// 20-frequency tile of 150 layers took 0.37 ms per step with the series against 0.21 ms without.)
+// Direct -> series, 10000 lines unless said: FP64 300 layers x 130 columns 458 -> 430 us, x 200
+// 577 -> 432, x 256 611 -> 449, 100 x 130 x 800 lines 59 -> 108 us; FP32 300 x 256 329 -> 381, 300 x 400
+// 425 -> 386 (7 tiles), 800 x 300 x 20000 lines 1632 -> 968.
 constexpr size_t kSeriesMaxWorkspace = size_t(4) << 30;
 constexpr int kSeriesMinTiles = 4;
-static bool series_on(const AlphaArgs &A, const rbx_launch &L) {
+static bool series_on(const AlphaArgs &A, const rbx_launch &L, int precision) {
     const int t = L.alpha_series;
-    return t == 2 || (t != 1 && A.tiles_total >= kSeriesMinTiles);
+    if (t != 0) return t == 2;
+    const int width = 64 * alpha_tile_k(A.nf, L);
+    if ((A.nf + width - 1) / width >= kSeriesMinTiles) return true;
+    const DevBlock *blk = A.cat.blk;
+    const long long lines = (A.abs.h2o ? blk[RBX_LINES_H2O].n : 0) +
+                            (nh3_has_hs(A.abs.nh3) ? blk[RBX_LINES_NH3_INV].n : 0);   // (the rest: about 1000)
+    const double terms = static_cast<double>(A.nl) * A.nf * lines;
+    return precision == RBX_FP64 ? A.nf > 128 && terms > 4e8 : A.nf > 256 && terms > 2e9;
 }
 
 // near-mask streams: one bit per line of every staging round of each selected segment
@@ -1806,12 +1825,14 @@ static int plan_alpha(AlphaArgs &A, const rbx_launch &L, int precision, int &K, 
                       size_t &bytes) {
     K = alpha_tile_k(A.nf, L);
     set_wave_tiles(A, K);
-    series = series_on(A, L);
+    series = series_on(A, L, precision);
     if (series) {
         far_layout(A);
         series = A.far_words > 0;   // no line lists selected: the plain path (one part)
     }
     if (series) {
+        K = series_tile_k(A, L);
+        set_wave_tiles(A, K);
         A.far_split = far_split(A, L);
         nsplit = 1;
         // the moments and near masks grow with layers x tiles x lines: past
@@ -1821,6 +1842,8 @@ static int plan_alpha(AlphaArgs &A, const rbx_launch &L, int precision, int &K, 
             series = false;
     }
     if (!series) {
+        K = alpha_tile_k(A.nf, L);
+        set_wave_tiles(A, K);
         int rc = alpha_split(A, L, K, precision, nsplit);
         if (rc) return rc;
     }
