@@ -131,6 +131,8 @@ class Alpha:
 
     def scale_table(self, scale, N):
         """(7, nl) per-constituent scale factors in RBX_C_* order for rbx_alpha."""
+        if not isinstance(scale, (dict, list, np.ndarray)):   # one factor for every layer
+            return np.full((len(_lib.CONSTITUENTS), N), float(scale) if utils.isanynum(scale) else 1.0)
         ls = self.get_layer_scale(scale, N)
         out = np.ones((len(_lib.CONSTITUENTS), N))
         for lyr, s in enumerate(ls):

@@ -72,16 +72,16 @@ class Brightness:
         Tb = np.empty((rays.shape[0], alpha.table.shape[1]))
         point = [i for i, d in enumerate(disc) if not d]
         if point:
-            sel = torch.as_tensor(point, device=hds.device)
+            h, n = _rows(hds, ns, point)
             # frequencies in the order they pass the cut (a fixed ~0.07 ms that saves ~10 % of
             # the integration): for large batches only
             big = len(point) * alpha.table.shape[1] >= ORDER_MIN_RAY_FREQS
-            Tb[point] = kernels.integrate(alpha.table, T, hds[sel], ns[sel], precision=prec,
+            Tb[point] = kernels.integrate(alpha.table, T, h, n, precision=prec,
                                           tau_cut=tau_cut, ordered=big).cpu().numpy()
         discs = [i for i, d in enumerate(disc) if d]
         if discs:
-            sel = torch.as_tensor(discs, device=hds.device)
-            Tb[discs] = kernels.integrate(alpha.table, T, hds[sel], ns[sel], disc=True,
+            h, n = _rows(hds, ns, discs)
+            Tb[discs] = kernels.integrate(alpha.table, T, h, n, disc=True,
                                           precision=prec).cpu().numpy()
         self.nsteps = ns.cpu().numpy()
         return Tb
@@ -125,3 +125,11 @@ class Brightness:
                 if not self.Tb[j] == utils.T_cmb and self.integrated_W[j] < 0.96:
                     print("Weight correction at {:.2f} is {:.4f} (showing below 0.96)".format(f, self.integrated_W[j]))
         return self.Tb
+
+
+def _rows(hds, ns, which):
+    """The paths of rays `which` (ascending); all of them without a copy."""
+    if len(which) == hds.shape[0]:
+        return hds, ns
+    sel = torch.as_tensor(which, device=hds.device)
+    return hds[sel], ns[sel]

@@ -18,9 +18,12 @@ NH3_MODELS = {'nh3_hs_sjs': 1, 'nh3_hs': 2, 'nh3_sjs': 3, 'nh3_dbs_sjs': 4, 'nh3
 
 
 def device():
-    if not torch.cuda.is_available():
-        raise RuntimeError('radiobear_amd needs a HIP device (torch.cuda.is_available() is False)')
-    return torch.device('cuda', torch.cuda.current_device())
+    try:   # (asking is_available() each time costs more than the rest of a small call's checks)
+        return torch.device('cuda', torch.cuda.current_device())
+    except (RuntimeError, AssertionError) as e:
+        if torch.cuda.is_available():
+            raise
+        raise RuntimeError('radiobear_amd needs a HIP device (torch.cuda.is_available() is False)') from e
 
 
 def _stream():
@@ -38,6 +41,24 @@ def as_device(x, dtype=torch.float64):
     else:
         t = torch.as_tensor(np.asarray(x), dtype=dtype, device=device())
     return t.contiguous()
+
+
+def as_device_all(*xs):
+    """as_device of each; host arrays cross in one copy (a copy from pageable memory costs about
+    20 us whatever its size), each then starting at a multiple of 512 bytes as tensors do."""
+    host = [i for i, x in enumerate(xs) if not isinstance(x, torch.Tensor)]
+    if len(host) < 2:
+        return [as_device(x) for x in xs]
+    arrays = [np.asarray(xs[i], dtype=np.float64) for i in host]
+    at = np.concatenate([[0], np.cumsum([-(-a.size // 64) * 64 for a in arrays])])
+    packed = np.zeros(int(at[-1]))
+    for k, a in zip(at, arrays):
+        packed[k:k + a.size] = a.ravel()
+    dev = as_device(packed)
+    out = list(xs)
+    for i, k, a in zip(host, at, arrays):
+        out[i] = dev[int(k):int(k) + a.size].view(a.shape)
+    return [as_device(x) for x in out]
 
 
 _CONSTS = {}          # small host arrays already copied to the device (request frequencies)
@@ -199,18 +220,15 @@ def cloud_table(cloud, Cl):
 def _alpha_inputs(P, T, mix, freqs, scale):
     f = np.asarray(freqs, dtype=np.float64)
     order, nf_low = nh3_order(f)
-    P = as_device(P)
-    T = as_device(T)
-    mix = as_device(mix)
+    P, T, mix, *sc = as_device_all(P, T, mix, *([] if scale is None else [scale]))
     nl = P.shape[0]
     if T.shape != (nl,) or mix.shape != (len(_lib.SPECIES), nl):
         raise ValueError('shape mismatch: P {}, T {}, mix {}'.format(tuple(P.shape), tuple(T.shape),
                                                                      tuple(mix.shape)))
     fd = device_const(f)
     fn = None if np.array_equal(order, np.arange(len(f))) else device_const(f[order])
-    sc = None
-    if scale is not None:
-        sc = as_device(scale)
+    sc = sc[0] if sc else None
+    if sc is not None:
         if sc.shape != (len(_lib.CONSTITUENTS), nl):
             raise ValueError('scale must be ({}, {})'.format(len(_lib.CONSTITUENTS), nl))
     return P, T, mix, fd, fn, nf_low, sc, nl
@@ -343,8 +361,7 @@ def _rays(b):
 
 def raypaths(planet, R, N, b, units='half_cm'):
     """Ray paths for impact parameters b (nray, 2): (ds (nray, nl-1) float64, nsteps (nray,) int32)."""
-    R = as_device(R)
-    N = as_device(N)
+    R, N, b = as_device_all(R, N, b)
     b = _rays(b)
     nl = R.shape[0]
     nray = b.shape[0]
