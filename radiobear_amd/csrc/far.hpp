@@ -15,10 +15,10 @@
 // (a = 0: 15 terms carry it, with coefficients growing like (k + 1) p^k); far lines are
 // small next to the near ones, and the tables stay within 3e-7 of FP64 like the direct
 // FP32 sums.  On 800 layers x 1024 frequencies (0.3-300 GHz, 128-column tiles) about
-// 30 % of the (line, tile) pairs are neither: only those are summed per column.  (12
+// 30 % of the (line, tile) pairs are neither: only those go to the near pass.  (12
 // terms at 1/4 leave more near pairs, 33 %, and were 2 % slower overall.)  FP64 mode uses
 // the same 16 terms at ratio 0.15 (at most ~8e-12 of a far line's value) and sums its near
-// lines in FP64 from their (D, a, c, g, G), as the direct FP64 sums do.
+// lines in FP64 from their (D, a, c, g, G).
 //
 // alpha_prep_kernel (one thread per layer and deriver) first writes every layer's
 // coefficient derivers to the workspace; both passes below read them from there.
@@ -33,9 +33,10 @@
 // alpha_near_kernel (block = tile x layer, all four wavefronts on the tile's
 // columns): lists the tile's near lines from its masks, derives each listed line's
 // coefficients again from its catalogue row (the catalogue stays in L2; no per-layer copy
-// of the lines goes through HBM), sums them as the line-sum kernel does with the lines
-// split between the wavefronts, adds the wavefronts in order and the series of the summed
-// moments, and writes the same per-slot partials the finish kernel reads (one part).
+// of the lines goes through HBM), sums them at the nodes of column intervals they are well
+// away from and at the columns they are close to, with the lines split between the
+// wavefronts, adds the wavefronts in order and the series of the summed moments, and
+// writes the same per-slot partials the finish kernel reads (one part).
 
 constexpr int kFarTerms = 16;
 // pole ratio of a far line: 1/3 in FP32 mode, 0.15 in FP64 mode (at most ~8e-12 of a far
