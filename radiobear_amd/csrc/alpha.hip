@@ -115,6 +115,7 @@ struct AlphaArgs {
     double *by_c;
     int tiles_total;   // forward kernel: wavefront tiles of tile_width columns
     int tile_width;    // columns per tile
+    int line_shares;   // direct sums: wavefronts of a block that share a tile's lines (1, 2 or 4)
     double *value;     // tangent: alpha [nl][nf] (float64) or null
     double *ws;        // forward: partial line sums [kSlots][nsplit][nl][nf]
     double *ws_base;   // forward: partial h2o base terms [nsplit][nl]
@@ -496,7 +497,7 @@ __device__ __forceinline__ void sum_staged_f64(const ST &st, const int (&set)[K]
 template <int K, bool F32, class Prep>
 __device__ void line_sum(const DevBlock &B, const Prep *prep, int need, bool active, const int (&set)[K],
                          const double *scale, const double (&x)[K], double (&acc)[K], SharedFwd &sh, double &base,
-                         int lb, int le, const WaveRanges &rng, int var) {
+                         int lb, int le, const WaveRanges &rng, int var, int share, int shares) {
     float xf[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) xf[k] = static_cast<float>(x[k]);
@@ -552,16 +553,18 @@ __device__ void line_sum(const DevBlock &B, const Prep *prep, int need, bool act
         }
         __syncthreads();
         if (active) {
+            // this wavefront's share of the staged lines, in chunks of kSub
+            const int jb = cntp / kSub * share / shares * kSub, je = cntp / kSub * (share + 1) / shares * kSub;
             if constexpr (F32) {
                 if (uni)
-                    sum_staged_f32<K, true>(sh.s32, set, 0, cntp, x, xf, acc);
+                    sum_staged_f32<K, true>(sh.s32, set, jb, je, x, xf, acc);
                 else
-                    sum_staged_f32<K, false>(sh.s32, set, 0, cntp, x, xf, acc);
+                    sum_staged_f32<K, false>(sh.s32, set, jb, je, x, xf, acc);
             } else {
                 if (uni)
-                    sum_staged_f64<K, true>(sh.s64, set, 0, cntp, x, acc);
+                    sum_staged_f64<K, true>(sh.s64, set, jb, je, x, acc);
                 else
-                    sum_staged_f64<K, false>(sh.s64, set, 0, cntp, x, acc);
+                    sum_staged_f64<K, false>(sh.s64, set, jb, je, x, acc);
             }
         }
         __syncthreads();
@@ -810,7 +813,12 @@ __global__ __launch_bounds__(kThreads, K >= 4 ? 3 : 4) void alpha_lines_kernel(A
     const int part = blockIdx.y, nsplit = gridDim.y;
     const LayerT<double> L = layer_of(A, layer);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
-    const int t = bx * (kThreads / 64) + wave;
+    // One wavefront per tile; a request of one or two tiles gives a tile all of its block's
+    // wavefronts, or half of them, each with its share of the staged lines (they only helped to stage
+    // them before: 333 layers x 77 columns x 5000 lines 154 -> 132 us, 1000 layers x 6 columns
+    // 120 -> 88, 150 layers x 20 columns x 2000 lines 64 -> 45).
+    const int shares = K == 1 ? A.line_shares : 1, share = wave % shares;
+    const int t = bx * (kThreads / 64) + wave / shares;
     const bool active = t < A.tiles_total;                // the block's last wavefronts may have no columns
     const int c0 = bx * kThreads * K, c1 = min(c0 + kThreads * K, A.nf);   // the block's columns
     const int need_inv = (c0 < A.nf_low ? 1 : 0) | (c1 > A.nf_low ? 2 : 0);
@@ -883,10 +891,17 @@ __global__ __launch_bounds__(kThreads, K >= 4 ? 3 : 4) void alpha_lines_kernel(A
     double acc[K] = {};
     auto store = [&](int q) {
         if (touched & (1 << q)) {
+            if (K == 1 && shares > 1) {   // a tile's shares, added in order
+                sh.red[threadIdx.x] = acc[0];
+                __syncthreads();
+                if (share == 0)
+                    for (int w = 1; w < shares; ++w) acc[0] += sh.red[threadIdx.x + w * 64];
+                __syncthreads();   // (the next lines are staged over them)
+            }
             double *w = A.ws + (static_cast<size_t>(q) * nsplit + part) * plane + static_cast<size_t>(layer) * A.nf;
 #pragma unroll
             for (int k = 0; k < K; ++k)
-                if (ok[k]) w[col[k]] = acc[k];
+                if (ok[k] && share == 0) w[col[k]] = acc[k];
         }
 #pragma unroll
         for (int k = 0; k < K; ++k) acc[k] = 0.0;
@@ -897,7 +912,7 @@ __global__ __launch_bounds__(kThreads, K >= 4 ? 3 : 4) void alpha_lines_kernel(A
         H2oPrep<double> prep(L);
         const double s[2] = {F32 ? pow2_scale(prep.pref * blk[RBX_LINES_H2O].wscale) : 1.0, 1.0};
         double a2[K] = {};
-        line_sum<K, F32>(blk[RBX_LINES_H2O], &prep, 1, active, one, s, x, a2, sh, base, lb, le, rng, 0);
+        line_sum<K, F32>(blk[RBX_LINES_H2O], &prep, 1, active, one, s, x, a2, sh, base, lb, le, rng, 0, share, shares);
 #pragma unroll
         for (int k = 0; k < K; ++k) acc[k] = a2[k] / s[0];
         did_h2o = true;
@@ -907,7 +922,7 @@ __global__ __launch_bounds__(kThreads, K >= 4 ? 3 : 4) void alpha_lines_kernel(A
         H2sPrep<double> prep(L);
         const double s[2] = {F32 ? pow2_scale(prep.pref * blk[RBX_LINES_H2S].wscale) : 1.0, 1.0};
         double a2[K] = {};
-        line_sum<K, F32>(blk[RBX_LINES_H2S], &prep, 1, active, one, s, x, a2, sh, unused, lb, le, rng, 0);
+        line_sum<K, F32>(blk[RBX_LINES_H2S], &prep, 1, active, one, s, x, a2, sh, unused, lb, le, rng, 0, share, shares);
 #pragma unroll
         for (int k = 0; k < K; ++k) acc[k] = a2[k] / s[0];
     }
@@ -917,7 +932,7 @@ __global__ __launch_bounds__(kThreads, K >= 4 ? 3 : 4) void alpha_lines_kernel(A
         const double s[2] = {F32 ? pow2_scale(prep[0].pref * blk[RBX_LINES_NH3_INV].wscale) : 1.0,
                              F32 ? pow2_scale(prep[1].pref * blk[RBX_LINES_NH3_INV].wscale) : 1.0};
         double a2[K] = {};
-        line_sum<K, F32>(blk[RBX_LINES_NH3_INV], prep, need_inv, active, set, s, xn, a2, sh, unused, lb, le, rng, 1);
+        line_sum<K, F32>(blk[RBX_LINES_NH3_INV], prep, need_inv, active, set, s, xn, a2, sh, unused, lb, le, rng, 1, share, shares);
 #pragma unroll
         for (int k = 0; k < K; ++k) acc[k] += a2[k] / s[set[k]];
     }
@@ -925,7 +940,7 @@ __global__ __launch_bounds__(kThreads, K >= 4 ? 3 : 4) void alpha_lines_kernel(A
         RotPrep<double> prep(L);
         const double s[2] = {F32 ? pow2_scale(prep.pref * blk[RBX_LINES_NH3_ROT].wscale) : 1.0, 1.0};
         double a2[K] = {};
-        line_sum<K, F32>(blk[RBX_LINES_NH3_ROT], &prep, 1, active, one, s, xn, a2, sh, unused, lb, le, rng, 1);
+        line_sum<K, F32>(blk[RBX_LINES_NH3_ROT], &prep, 1, active, one, s, xn, a2, sh, unused, lb, le, rng, 1, share, shares);
 #pragma unroll
         for (int k = 0; k < K; ++k) acc[k] += a2[k] / s[0];
     }
@@ -933,7 +948,7 @@ __global__ __launch_bounds__(kThreads, K >= 4 ? 3 : 4) void alpha_lines_kernel(A
         V2Prep<double> prep(L);
         const double s[2] = {F32 ? pow2_scale(prep.pref * blk[RBX_LINES_NH3_V2].wscale) : 1.0, 1.0};
         double a2[K] = {};
-        line_sum<K, F32>(blk[RBX_LINES_NH3_V2], &prep, 1, active, one, s, xn, a2, sh, unused, lb, le, rng, 1);
+        line_sum<K, F32>(blk[RBX_LINES_NH3_V2], &prep, 1, active, one, s, xn, a2, sh, unused, lb, le, rng, 1, share, shares);
 #pragma unroll
         for (int k = 0; k < K; ++k) acc[k] += a2[k] / s[0];
     }
@@ -942,7 +957,7 @@ __global__ __launch_bounds__(kThreads, K >= 4 ? 3 : 4) void alpha_lines_kernel(A
         Ph3Prep<double> prep(L);
         const double s[2] = {F32 ? pow2_scale(prep.pref * blk[RBX_LINES_PH3].wscale) : 1.0, 1.0};
         double a2[K] = {};
-        line_sum<K, F32>(blk[RBX_LINES_PH3], &prep, 1, active, one, s, x, a2, sh, unused, lb, le, rng, 0);
+        line_sum<K, F32>(blk[RBX_LINES_PH3], &prep, 1, active, one, s, x, a2, sh, unused, lb, le, rng, 0, share, shares);
 #pragma unroll
         for (int k = 0; k < K; ++k) acc[k] = a2[k] / s[0];
     }
@@ -1844,6 +1859,9 @@ static int plan_alpha(AlphaArgs &A, const rbx_launch &L, int precision, int &K, 
     if (!series) {
         K = alpha_tile_k(A.nf, L);
         set_wave_tiles(A, K);
+        // (a launch shape that names the tile width keeps a wavefront per tile: FP64 tables are then
+        // the same at every width)
+        A.line_shares = L.alpha_k != 0 || K != 1 || A.tiles_total > 2 ? 1 : 4 / A.tiles_total;
         int rc = alpha_split(A, L, K, precision, nsplit);
         if (rc) return rc;
     }
