@@ -172,7 +172,7 @@ typedef struct rbx_launch {
                            series (at most 8e-7 / 8e-12 of a far line's value: FP32 tables within
                            3e-7 of FP64 as the direct sums, FP64 tables within 1e-11 of the direct
                            FP64 sums); built in: 2 for requests of 4 or more wavefront tiles (fewer in
-                           FP64 past 128 frequencies, in FP32 past 256, when layers x lines are many) while
+                           FP64 past 160 frequencies, in FP32 past 256, when layers x lines are many) while
                            the workspace (the tiles' moments and near-line masks: about 0.1 MB per
                            layer at 1024 frequencies and 25553 lines) stays under 4 GiB, else 1 */
     int alpha_split;    /* parts each layer's direct line sums are split into: 1..16 (built in: a

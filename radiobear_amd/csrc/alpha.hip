@@ -873,6 +873,39 @@ __global__ __launch_bounds__(kThreads, K >= 4 ? 3 : 4) void alpha_lines_kernel(A
     const LinePlan plan(A, L.P);
     const int *nr = plan.nr;
     const int r0 = plan.begin(part, nsplit), r1 = plan.begin(part + 1, nsplit);
+    // The part's coefficient derivers, dealt to the wavefronts and kept in LDS with their weight scales:
+    // their two dozen FP64 powers are a wavefront's whole work for several hundred lines, and every
+    // wavefront used to form them all (1000 layers x 6 columns 88 -> 65 us, 150 x 20 x 2000 lines 45 -> 36,
+    // 333 x 77 x 5000 132 -> 110).
+    __shared__ __align__(16) double prep_at[kSegs + 1][8];
+    __shared__ double scale_at[kSegs + 1];
+    {
+        int at = 0, turn = 0;
+        auto form = [&](int slot, auto make, int kind) {   // the next wavefront's turn
+            if (turn++ % (kThreads / 64) != wave) return;
+            const auto p = make();
+            using Prep = std::decay_t<decltype(p)>;
+            static_assert(sizeof(Prep) <= sizeof(prep_at[0]), "a deriver is at most 8 doubles");
+            if (lane == 0) {
+                *reinterpret_cast<Prep *>(prep_at[slot]) = p;
+                scale_at[slot] = F32 ? pow2_scale(p.pref * A.cat.blk[kind].wscale) : 1.0;
+            }
+        };
+        auto here = [&](int s) {   // segment s has rounds in this part
+            const int a = at;
+            at += nr[s];
+            return max(r0, a) < min(r1, a + nr[s]);
+        };
+        const bool h2o = here(0), h2s = here(1), inv = here(2), rot = here(3), v2 = here(4), ph3 = here(5);
+        if (inv && (need_inv & 1)) form(2, [&] { return InvPrep<double>(L, nh3_low_set(A.abs.nh3)); }, RBX_LINES_NH3_INV);
+        if (inv && (need_inv & 2)) form(kSegs, [&] { return InvPrep<double>(L, 1); }, RBX_LINES_NH3_INV);
+        if (rot) form(3, [&] { return RotPrep<double>(L); }, RBX_LINES_NH3_ROT);
+        if (v2) form(4, [&] { return V2Prep<double>(L); }, RBX_LINES_NH3_V2);
+        if (h2o) form(0, [&] { return H2oPrep<double>(L); }, RBX_LINES_H2O);
+        if (h2s) form(1, [&] { return H2sPrep<double>(L); }, RBX_LINES_H2S);
+        if (ph3) form(5, [&] { return Ph3Prep<double>(L); }, RBX_LINES_PH3);
+    }
+    __syncthreads();
     int seg = 0, off = 0, lb = 0, le = 0;
     // lines [lb, le) of the next segment that fall in this part's rounds
     auto next = [&](int n) {
@@ -909,55 +942,57 @@ __global__ __launch_bounds__(kThreads, K >= 4 ? 3 : 4) void alpha_lines_kernel(A
     double base = 0.0, unused = 0.0;
     bool did_h2o = false;
     if (next(blk[RBX_LINES_H2O].n)) {
-        H2oPrep<double> prep(L);
-        const double s[2] = {F32 ? pow2_scale(prep.pref * blk[RBX_LINES_H2O].wscale) : 1.0, 1.0};
+        const auto *prep = reinterpret_cast<const H2oPrep<double> *>(prep_at[0]);
+        const double s[2] = {scale_at[0], 1.0};
         double a2[K] = {};
-        line_sum<K, F32>(blk[RBX_LINES_H2O], &prep, 1, active, one, s, x, a2, sh, base, lb, le, rng, 0, share, shares);
+        line_sum<K, F32>(blk[RBX_LINES_H2O], prep, 1, active, one, s, x, a2, sh, base, lb, le, rng, 0, share, shares);
 #pragma unroll
         for (int k = 0; k < K; ++k) acc[k] = a2[k] / s[0];
         did_h2o = true;
     }
     store(kSlotH2o);
     if (next(blk[RBX_LINES_H2S].n)) {
-        H2sPrep<double> prep(L);
-        const double s[2] = {F32 ? pow2_scale(prep.pref * blk[RBX_LINES_H2S].wscale) : 1.0, 1.0};
+        const auto *prep = reinterpret_cast<const H2sPrep<double> *>(prep_at[1]);
+        const double s[2] = {scale_at[1], 1.0};
         double a2[K] = {};
-        line_sum<K, F32>(blk[RBX_LINES_H2S], &prep, 1, active, one, s, x, a2, sh, unused, lb, le, rng, 0, share, shares);
+        line_sum<K, F32>(blk[RBX_LINES_H2S], prep, 1, active, one, s, x, a2, sh, unused, lb, le, rng, 0, share, shares);
 #pragma unroll
         for (int k = 0; k < K; ++k) acc[k] = a2[k] / s[0];
     }
     store(kSlotH2s);
     if (next(blk[RBX_LINES_NH3_INV].n)) {
-        const InvPrep<double> prep[2] = {InvPrep<double>(L, nh3_low_set(A.abs.nh3)), InvPrep<double>(L, 1)};
-        const double s[2] = {F32 ? pow2_scale(prep[0].pref * blk[RBX_LINES_NH3_INV].wscale) : 1.0,
-                             F32 ? pow2_scale(prep[1].pref * blk[RBX_LINES_NH3_INV].wscale) : 1.0};
+        // (set 0's weights serve both sets: they are the same in either deriver)
+        const int first = (need_inv & 1) ? 2 : kSegs, second = (need_inv & 2) ? kSegs : 2;
+        const InvPrep<double> prep[2] = {*reinterpret_cast<const InvPrep<double> *>(prep_at[first]),
+                                         *reinterpret_cast<const InvPrep<double> *>(prep_at[second])};
+        const double s[2] = {scale_at[first], scale_at[second]};
         double a2[K] = {};
         line_sum<K, F32>(blk[RBX_LINES_NH3_INV], prep, need_inv, active, set, s, xn, a2, sh, unused, lb, le, rng, 1, share, shares);
 #pragma unroll
         for (int k = 0; k < K; ++k) acc[k] += a2[k] / s[set[k]];
     }
     if (next(blk[RBX_LINES_NH3_ROT].n)) {
-        RotPrep<double> prep(L);
-        const double s[2] = {F32 ? pow2_scale(prep.pref * blk[RBX_LINES_NH3_ROT].wscale) : 1.0, 1.0};
+        const auto *prep = reinterpret_cast<const RotPrep<double> *>(prep_at[3]);
+        const double s[2] = {scale_at[3], 1.0};
         double a2[K] = {};
-        line_sum<K, F32>(blk[RBX_LINES_NH3_ROT], &prep, 1, active, one, s, xn, a2, sh, unused, lb, le, rng, 1, share, shares);
+        line_sum<K, F32>(blk[RBX_LINES_NH3_ROT], prep, 1, active, one, s, xn, a2, sh, unused, lb, le, rng, 1, share, shares);
 #pragma unroll
         for (int k = 0; k < K; ++k) acc[k] += a2[k] / s[0];
     }
     if (next(blk[RBX_LINES_NH3_V2].n)) {
-        V2Prep<double> prep(L);
-        const double s[2] = {F32 ? pow2_scale(prep.pref * blk[RBX_LINES_NH3_V2].wscale) : 1.0, 1.0};
+        const auto *prep = reinterpret_cast<const V2Prep<double> *>(prep_at[4]);
+        const double s[2] = {scale_at[4], 1.0};
         double a2[K] = {};
-        line_sum<K, F32>(blk[RBX_LINES_NH3_V2], &prep, 1, active, one, s, xn, a2, sh, unused, lb, le, rng, 1, share, shares);
+        line_sum<K, F32>(blk[RBX_LINES_NH3_V2], prep, 1, active, one, s, xn, a2, sh, unused, lb, le, rng, 1, share, shares);
 #pragma unroll
         for (int k = 0; k < K; ++k) acc[k] += a2[k] / s[0];
     }
     store(kSlotNh3);
     if (next(blk[RBX_LINES_PH3].n)) {
-        Ph3Prep<double> prep(L);
-        const double s[2] = {F32 ? pow2_scale(prep.pref * blk[RBX_LINES_PH3].wscale) : 1.0, 1.0};
+        const auto *prep = reinterpret_cast<const Ph3Prep<double> *>(prep_at[5]);
+        const double s[2] = {scale_at[5], 1.0};
         double a2[K] = {};
-        line_sum<K, F32>(blk[RBX_LINES_PH3], &prep, 1, active, one, s, x, a2, sh, unused, lb, le, rng, 0, share, shares);
+        line_sum<K, F32>(blk[RBX_LINES_PH3], prep, 1, active, one, s, x, a2, sh, unused, lb, le, rng, 0, share, shares);
 #pragma unroll
         for (int k = 0; k < K; ++k) acc[k] = a2[k] / s[0];
     }
@@ -1717,9 +1752,9 @@ static int alpha_split(const AlphaArgs &A, const rbx_launch &L, int K, int preci
 // kSeriesMaxWorkspace for requests of at least kSeriesMinTiles tiles of the direct sums' width, and of
 // fewer where the direct sums are long enough that the two passes' launches (about 50 us) pay.  (One
 // 20-frequency tile of 150 layers took 0.37 ms per step with the series against 0.21 ms without.)
-// Direct -> series, 10000 lines unless said: FP64 300 layers x 130 columns 458 -> 430 us, x 200
-// 577 -> 432, x 256 611 -> 449, 100 x 130 x 800 lines 59 -> 108 us; FP32 300 x 256 329 -> 381, 300 x 400
-// 425 -> 386 (7 tiles), 800 x 300 x 20000 lines 1632 -> 968.
+// Direct -> series, 10000 lines unless said: FP64 300 layers x 130 columns 419 -> 430 us, x 200
+// 528 -> 432, x 256 581 -> 450, 100 x 130 x 800 lines 53 -> 110 us; FP32 300 x 256 305 -> 381, 300 x 400
+// 425 -> 386 (7 tiles), 800 x 300 x 20000 lines 1522 -> 968.
 constexpr size_t kSeriesMaxWorkspace = size_t(4) << 30;
 constexpr int kSeriesMinTiles = 4;
 static bool series_on(const AlphaArgs &A, const rbx_launch &L, int precision) {
@@ -1731,7 +1766,7 @@ static bool series_on(const AlphaArgs &A, const rbx_launch &L, int precision) {
     const long long lines = (A.abs.h2o ? blk[RBX_LINES_H2O].n : 0) +
                             (nh3_has_hs(A.abs.nh3) ? blk[RBX_LINES_NH3_INV].n : 0);   // (the rest: about 1000)
     const double terms = static_cast<double>(A.nl) * A.nf * lines;
-    return precision == RBX_FP64 ? A.nf > 128 && terms > 4e8 : A.nf > 256 && terms > 2e9;
+    return precision == RBX_FP64 ? A.nf > 160 && terms > 4e8 : A.nf > 256 && terms > 2e9;
 }
 
 // near-mask streams: one bit per line of every staging round of each selected segment
