@@ -49,7 +49,8 @@ constexpr int kFarMom = kFarSets * 2 * kFarTerms;     // moments per (layer, par
 constexpr int kSegStream[kSegs] = {0, 1, 2, 4, 5, 6};
 constexpr int kSegFarSet[kSegs] = {0, 1, 2, 4, 4, 5};
 constexpr int kSegVar[kSegs] = {0, 0, 1, 1, 1, 0};    // columns' x (0) or x for NH3 (1)
-constexpr int kListWords = 128;                       // mask words listed per window
+constexpr int kListWords = 112;                       // mask words listed per window (near_sum; with 128 the
+                                                      // widest FP32 tile's block is past a quarter of a CU's LDS)
 constexpr int kFarRanges = 4;                         // x; x NH3; x NH3 of set 0 columns; of set 1
 
 __device__ inline void tile_cols(const AlphaArgs &A, int tile, int &c0, int &c1) {
@@ -562,9 +563,18 @@ __global__ __launch_bounds__(kThreads, 3) void alpha_far_kernel(AlphaArgs args) 
 // f but for its poles +-sqrt(p), so over an interval of columns [lo, hi] that lies well away from
 // them it is its Chebyshev interpolant on n nodes to rho^-n, rho the Bernstein ellipse (foci lo
 // and hi) through the nearest pole: n values stand for all the interval's columns.  Lines outside
-// rho = 3.2 are taken at nodes: 16 in FP32 mode (8e-9 of the line's value, below an FP32 term's
-// roundings), 32 in FP64 mode (7e-17; 16 nodes outside rho = 6, 4e-13, took the same time and left
-// tables 1e-13 to 3e-13 from 64 bits where the direct sums leave 1e-15).
+// rho are taken at nodes.  The rate alone does not give the error: a narrow line's two conjugate poles
+// all but cancel (a near-double pole, n rho^-n), and its value at a far column is up to 13 times less
+// than at the interval's near end.  For lines of every form with their pole on the ellipse, the worst
+// error relative to the line's own value at the column, and to its largest in the interval:
+//   16 nodes  rho 3.2: 3.5e-6, 2.5e-7   4.0: 8.7e-8, 1.2e-8   4.2: 4.6e-8, 6.3e-9
+//   32 nodes  rho 3.2: 4.2e-14, 4e-15   3.6: 1.0e-15, 1.2e-16
+// FP32 mode takes 16 nodes outside 4.2 (under one FP32 rounding, 6e-8), FP64 mode 32 outside 3.6 (the
+// roundings of an FP64 term).
+//
+// A node's value reaches every column of its interval, so the node sums are FP64 in FP32 mode too:
+// FP32 ones left tables 7 % (rms over 90 requests; at worst 25 %) further from FP64 than sums at
+// every column, FP64 ones 6 % nearer.  At a leaf's columns FP32 mode sums as sum_staged_f32 does.
 //
 // The tile's columns form a binary tree of intervals (whole tile, halves, ... down to leaves of 32
 // columns, 64 in FP64 mode).  A batch of 64 listed lines (neighbours in frequency, so they mostly
@@ -572,14 +582,13 @@ __global__ __launch_bounds__(kThreads, 3) void alpha_far_kernel(AlphaArgs args) 
 // nodes, and a leaf that some line is close to at its columns.  Lanes are the points of one interval
 // times groups of lines: 4 groups at 16 nodes, 2 at 32 points.  The sums stay per interval until the
 // slot's last line; then their Chebyshev coefficients are formed and each column adds its ancestors'
-// series.  By points, 128-column tiles of 1024 columns over 0.3-300 GHz need about 95 (FP32) where
-// every column of every listed line was 250 per line and unit of ln f; what remains is half the
-// direct points' FP64 detunings and half deriving the listed lines and finding their intervals.
-// The pass, before -> now: 400 layers x 512 columns x 11000 lines 331 -> 208 us (FP32), 812 -> 332
-// (FP64); 800 x 1024 x 25553 1517 -> 1067, 4195 -> 1936; 600 x 1000 x 11000 FP64 1569 -> 725; 300 x 201
-// FP64 421 -> 231.  Four wavefronts per SIMD (about 100 B of scratch a lane) against three without:
-// 800 x 1024 1575 against 1771 us for the whole table (FP32), five 1502 but 256-column tiles slower.
-constexpr double kNodeRho = 3.2;
+// series.  Every column of every listed line against this, the pass alone: 400 layers x 512 columns x
+// 11000 lines 331 -> 243 us (FP32), 812 -> 342 (FP64); 800 x 1024 x 26000 1517 -> 1171, 4195 -> 1882;
+// 600 x 1000 x 11000 FP64 1569 -> 639; 300 x 201 FP64 421 -> 237.  (FP32 node sums outside rho = 3.2
+// took 208 and 1067 us in FP32 mode.)  It is held at four wavefronts per SIMD (about 100 B of scratch a
+// lane): 800 x 1024 x 26000, FP32, the whole request 2.85 ms with three, 2.64-2.78 with four.
+template <bool F32>
+__host__ __device__ constexpr double node_rho() { return F32 ? 4.2 : 3.6; }
 
 template <int K, bool F32>
 struct NearTree {
@@ -632,8 +641,10 @@ constexpr int kWaveBatch = 64;
 struct WaveStage {
     alignas(16) double D[kWaveBatch];    // Ds
     alignas(16) double h[kWaveBatch];
-    alignas(16) float2 ac[kWaveBatch];   // a, c (scaled)
-    alignas(16) float2 dh[kWaveBatch];   // Ds less the interval's x centre, and h, rounded to FP32
+    alignas(16) double a[kWaveBatch];    // a, c (scaled)
+    alignas(16) double c[kWaveBatch];
+    alignas(16) float2 ac[kWaveBatch];   // a, c and Ds, h rounded to FP32
+    alignas(16) float2 dh[kWaveBatch];
 };
 
 // FP64 mode: the (D, a, c, g, G) of the direct FP64 sums
@@ -685,8 +696,8 @@ __device__ inline double far_eval(const double *mom, double x) {
 }
 
 // A listed line's coefficients for the near sums, derived from its catalogue row as pass 1
-// derives them, with the segment's coefficient sets read from LDS: FP32 (Ds, h, a s, c s),
-// FP64 (D, a, c, g, G)
+// derives them, with the segment's coefficient sets read from LDS: FP32 mode (Ds, h, a s, c s),
+// FP64 mode (D, a, c, g, G)
 template <class Prep, int NC>
 __device__ __forceinline__ CoefT<double> near_coef(const DevBlock &B, int i, int v, const double (&prep)[2][8]) {
     LineRow<NC> row;
@@ -698,7 +709,7 @@ __device__ __forceinline__ CoefT<double> near_coef(const DevBlock &B, int i, int
 
 template <bool F32>
 __device__ __forceinline__ void derive_near(int seg, int v, const DevBlock &B, int i, const double (&prep)[2][8],
-                                            double sv, double (&c5)[5], float2 &ac) {
+                                            double sv, double (&c5)[5]) {
     CoefT<double> c;
     switch (seg) {
         case 0: c = near_coef<H2oPrep<double>, kNumCols[RBX_LINES_H2O]>(B, i, v, prep); break;
@@ -710,7 +721,8 @@ __device__ __forceinline__ void derive_near(int seg, int v, const DevBlock &B, i
     }
     if constexpr (F32) {
         shifted_denominator(c, c5[0], c5[1]);
-        ac = make_float2(static_cast<float>(c.a * sv), static_cast<float>(c.c * sv));
+        c5[2] = c.a * sv;
+        c5[3] = c.c * sv;
     } else {
         c5[0] = c.D;
         c5[1] = c.a;
@@ -754,13 +766,44 @@ __device__ __forceinline__ bool outside(const float2 &z, const NearInterval &I) 
 }
 
 // Sum of the staged lines' terms at this lane's point x, over the pairs of lines g, g + G, ... of
-// the batch's first `npairs` (a multiple of 4 G), two lines over one denominator and blocks of 8
-// lines in FP32.  `fast`: bit j = lines [8 j, 8 j + 8) take the all-FP32 denominator
-// (dx - dD)^2 + h, dx and dD the distances of x and Ds from the interval's centre; the others form
-// it in FP64 (as sum_staged_f32).
+// the batch's first `npairs` (a multiple of 4 G), two lines over one denominator: in FP64 from
+// (Ds, h, a, c) ...
 template <int G>
-__device__ __forceinline__ double sum_pairs(const WaveStage &st, int g, int npairs, double x, float dx,
-                                            unsigned int fast) {
+__device__ __forceinline__ double sum_pairs(const WaveStage &st, int g, int npairs, double x) {
+    double acc = 0.0;
+#pragma unroll 2
+    for (int p = g; p < npairs; p += G) {
+        const double2 D = reinterpret_cast<const double2 *>(st.D)[p], h = reinterpret_cast<const double2 *>(st.h)[p];
+        const double2 a = reinterpret_cast<const double2 *>(st.a)[p], c = reinterpret_cast<const double2 *>(st.c)[p];
+        const double d1 = x - D.x, d2 = x - D.y;
+        const double n1 = fma(a.x, x, c.x), n2 = fma(a.y, x, c.y);
+        const double e1 = fma(d1, d1, h.x), e2 = fma(d2, d2, h.y);
+        acc += fma(n1, e2, n2 * e1) * recip(e1 * e2);
+    }
+    return acc;
+}
+
+// ... and from (D, a, c, g, G), the terms of sum_staged_f64
+template <int G>
+__device__ __forceinline__ double sum_pairs(const WaveStage64 &st, int g, int npairs, double x) {
+    double acc = 0.0;
+#pragma unroll 2
+    for (int p = g; p < npairs; p += G) {
+        const double2 D = reinterpret_cast<const double2 *>(st.D)[p], a = reinterpret_cast<const double2 *>(st.a)[p];
+        const double2 c = reinterpret_cast<const double2 *>(st.c)[p], gg = reinterpret_cast<const double2 *>(st.g)[p];
+        const double2 GG = reinterpret_cast<const double2 *>(st.G)[p];
+        const double d1 = x - D.x, d2 = x - D.y;
+        const double n1 = fma(a.x, x, c.x), n2 = fma(a.y, x, c.y);
+        const double e1 = fma(d1, d1, fma(gg.x, x, GG.x)), e2 = fma(d2, d2, fma(gg.y, x, GG.y));
+        acc += fma(n1, e2, n2 * e1) * recip(e1 * e2);
+    }
+    return acc;
+}
+
+// The same at a column in FP32 mode (sum_staged_f32), blocks of 8 lines in FP32.  `fast`: bit j = lines
+// [8 j, 8 j + 8) are FP32-safe for the tile's columns; the others form their denominators in FP64.
+template <int G>
+__device__ __forceinline__ double sum_pairs_f32(const WaveStage &st, int g, int npairs, double x, unsigned int fast) {
     const float xf = static_cast<float>(x);
     constexpr unsigned int kAll = (1u << G) - 1u;
     double acc = 0.0;
@@ -771,7 +814,7 @@ __device__ __forceinline__ double sum_pairs(const WaveStage &st, int g, int npai
             for (int u = 0; u < 4; ++u) {
                 const float4 dp = reinterpret_cast<const float4 *>(st.dh)[p0 + u * G + g];
                 const float4 qp = reinterpret_cast<const float4 *>(st.ac)[p0 + u * G + g];
-                const float d1 = dx - dp.x, d2 = dx - dp.z;
+                const float d1 = xf - dp.x, d2 = xf - dp.z;
                 const float e1 = fmaf(d1, d1, dp.y), e2 = fmaf(d2, d2, dp.w);
                 const float n1 = fmaf(qp.x, xf, qp.y), n2 = fmaf(qp.z, xf, qp.w);
                 p = fmaf(fmaf(n2, e1, n1 * e2), __builtin_amdgcn_rcpf(e1 * e2), p);
@@ -793,32 +836,14 @@ __device__ __forceinline__ double sum_pairs(const WaveStage &st, int g, int npai
     return acc;
 }
 
-// the same in FP64 (the terms of sum_staged_f64)
-template <int G>
-__device__ __forceinline__ double sum_pairs(const WaveStage64 &st, int g, int npairs, double x, float, unsigned int) {
-    double acc = 0.0;
-#pragma unroll 2
-    for (int p = g; p < npairs; p += G) {
-        const double2 D = reinterpret_cast<const double2 *>(st.D)[p], a = reinterpret_cast<const double2 *>(st.a)[p];
-        const double2 c = reinterpret_cast<const double2 *>(st.c)[p], gg = reinterpret_cast<const double2 *>(st.g)[p];
-        const double2 GG = reinterpret_cast<const double2 *>(st.G)[p];
-        const double d1 = x - D.x, d2 = x - D.y;
-        const double n1 = fma(a.x, x, c.x), n2 = fma(a.y, x, c.y);
-        const double e1 = fma(d1, d1, fma(gg.x, x, GG.x)), e2 = fma(d2, d2, fma(gg.y, x, GG.y));
-        acc += fma(n1, e2, n2 * e1) * recip(e1 * e2);
-    }
-    return acc;
-}
-
-// A batch's staged lines added at the tree's points: this lane's line has shifted centre Ds, h and
-// pole z (`line` false: padding, a zero term); columns' x of the leaves from `colx`.
+// A batch's staged lines added at the tree's points: this lane's line has pole z (`line` false:
+// padding, a zero term); `fast` as for sum_pairs_f32; columns' x of the leaves from `colx`.
 template <int K, bool F32, class ColX>
-__device__ __forceinline__ void sum_tree(NearShared<K, F32> &sh, int rv, bool line, double Ds, double h, int count,
-                                         double inv_scale, const ColX &colx) {
+__device__ __forceinline__ void sum_tree(NearShared<K, F32> &sh, int rv, bool line, const float2 &z, unsigned int fast,
+                                         int count, double inv_scale, const ColX &colx) {
     using Tree = NearTree<K, F32>;
     const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-    auto &st = sh.st[wave];
-    const float2 z = pole_in_f(Ds, h);
+    const auto &st = sh.st[wave];
     const double node = sh.cosines[(2 * (lane % Tree::nodes) + 1) * (kCosTab / 4 / Tree::nodes)];
     unsigned int pending = 2u;
 #pragma unroll 1
@@ -831,34 +856,22 @@ __device__ __forceinline__ void sum_tree(NearShared<K, F32> &sh, int rv, bool li
             pending |= 3u << (2 * i);
             continue;
         }
-        const double xc = I.c * I.c;
-        unsigned int fast = 0u;
-        if constexpr (F32) {
-            // FP32 denominators: the distances' roundings stay within a few of x - Ds (or of the
-            // root of h beside it) past twice the interval's half width in x, as they do for every
-            // line outside the ellipse; h < 0 must not cancel (x - Ds)^2
-            const double dD = Ds - xc, lo2 = static_cast<double>(I.lo) * I.lo - Ds;
-            const float rx = static_cast<float>(I.r * (2.0 * I.c + I.r)), dDf = static_cast<float>(dD);
-            const bool ok = h >= 0.0 ? (nodes || fabsf(dDf) >= 2.0f * rx || static_cast<float>(h) >= rx * rx)
-                                     : (lo2 > 0.0 && lo2 * lo2 >= -4.0 * h && (nodes || fabsf(dDf) >= 2.0f * rx));
-            fast = full_chunks(__ballot(!line || ok));
-            wave_sync();   // (the interval before has been summed)
-            st.dh[lane] = make_float2(dDf, static_cast<float>(h));
-            wave_sync();
-        }
         if (nodes) {
             constexpr int G = Tree::node_groups;
-            const double f = fma(I.r, node, I.c), x = f * f;
-            const double s = group_sum<G>(sum_pairs<G>(st, lane / Tree::nodes, (count + 8 * G - 1) / (8 * G) * (4 * G), x,
-                                                       static_cast<float>(x - xc), fast));
+            const double f = fma(I.r, node, I.c);
+            const double s = group_sum<G>(sum_pairs<G>(st, lane / Tree::nodes, (count + 8 * G - 1) / (8 * G) * (4 * G), f * f));
             double &v = sh.node[wave][i][lane % Tree::nodes];
             if (lane < Tree::nodes) v = fma(s, inv_scale, v);
         } else {
             constexpr int G = Tree::col_groups;
             const int k = (i - Tree::leaves) * Tree::width + lane % Tree::width;
-            const double x = colx(k);
-            const double s = group_sum<G>(sum_pairs<G>(st, lane / Tree::width, (count + 8 * G - 1) / (8 * G) * (4 * G), x,
-                                                       static_cast<float>(x - xc), fast));
+            const int npairs = (count + 8 * G - 1) / (8 * G) * (4 * G);
+            double s;
+            if constexpr (F32)
+                s = sum_pairs_f32<G>(st, lane / Tree::width, npairs, colx(k), fast);
+            else
+                s = sum_pairs<G>(st, lane / Tree::width, npairs, colx(k));
+            s = group_sum<G>(s);
             double &v = sh.column[wave][k];
             if (lane < Tree::width) v = fma(s, inv_scale, v);
         }
@@ -896,20 +909,25 @@ __device__ void near_sum(int n, const Derive &derive, int rv, const unsigned int
         if (total > 0 && tid == 0) sh.used = 1;
         __syncthreads();
         // listed line e's coefficients, derived from its catalogue row when its batch is
-        // staged (past the list: a zero term): FP32 (Ds, h, a s, c s), FP64 (D, a, c, g, G)
+        // staged (past the list: a zero term): FP32 mode (Ds, h, a s, c s), FP64 mode (D, a, c, g, G)
         const int nb = (total + kWaveBatch - 1) / kWaveBatch;
         for (int b = wave; b < nb; b += kThreads / 64) {
             const int e = b * kWaveBatch + lane;
             const int i = e < total ? w0 * 32 + sh.list[e] : n;
             double c5[5] = {0.0, F32 ? 1.0 : 0.0, 0.0, 0.0, 1.0};
-            float2 ac = make_float2(0.0f, 0.0f);
-            if (i < n) derive(i, c5, ac);
+            if (i < n) derive(i, c5);
             double Ds = c5[0], h = c5[1];
+            unsigned int fast = 0u;
             wave_sync();   // (the batch before has been summed)
             if constexpr (F32) {
+                const double lo = sh.iv[rv][1].lo, hi = sh.iv[rv][1].hi;
                 st.D[lane] = Ds;
                 st.h[lane] = h;
-                st.ac[lane] = ac;
+                st.a[lane] = c5[2];
+                st.c[lane] = c5[3];
+                st.ac[lane] = make_float2(static_cast<float>(c5[2]), static_cast<float>(c5[3]));
+                st.dh[lane] = make_float2(static_cast<float>(Ds), static_cast<float>(h));
+                fast = full_chunks(__ballot(lo >= 0.0 && fp32_safe(Ds, h, lo * lo, hi * hi)));
             } else {
                 st.D[lane] = c5[0];
                 st.a[lane] = c5[1];
@@ -919,7 +937,8 @@ __device__ void near_sum(int n, const Derive &derive, int rv, const unsigned int
                 shifted_denominator(CoefT<double>{c5[0], c5[1], c5[2], c5[3], c5[4]}, Ds, h);
             }
             wave_sync();
-            sum_tree<K, F32>(sh, rv, i < n, Ds, h, min(kWaveBatch, total - b * kWaveBatch), inv_scale, colx);
+            sum_tree<K, F32>(sh, rv, i < n, pole_in_f(Ds, h), fast, min(kWaveBatch, total - b * kWaveBatch), inv_scale,
+                             colx);
         }
         __syncthreads();   // every wavefront is done with this window's list
     }
@@ -1045,7 +1064,7 @@ __global__ __launch_bounds__(kThreads, 4) void alpha_near_kernel(AlphaArgs args)
         // node's f is rounded to 2^-53 c, which moves a term by up to about 2^-53 c / r of itself:
         // FP64 mode takes no nodes in narrow intervals.
         const bool use = lo >= 0.0 && (F32 || 64.0 * I.r >= I.c);
-        I.thr = use ? static_cast<float>(I.r * (kNodeRho + 1.0 / kNodeRho) + 1.0e-6 * hi) : INFINITY;
+        I.thr = use ? static_cast<float>(I.r * (node_rho<F32>() + 1.0 / node_rho<F32>()) + 1.0e-6 * hi) : INFINITY;
     }
     for (int e = tid; e < kFarMom; e += kThreads) {
         double s = 0.0;
@@ -1112,7 +1131,7 @@ __global__ __launch_bounds__(kThreads, 4) void alpha_near_kernel(AlphaArgs args)
                 if (inv ? !((tsets >> v) & 1) : v > 0) continue;
                 const unsigned int *mk = masks + A.far_off[kSegStream[seg] + (inv ? v : 0)];
                 const double sv = sh.scale[v];
-                auto derive = [&](int i, double (&c5)[5], float2 &ac) { derive_near<F32>(seg, v, B, i, sh.prep, sv, c5, ac); };
+                auto derive = [&](int i, double (&c5)[5]) { derive_near<F32>(seg, v, B, i, sh.prep, sv, c5); };
                 const int rv = inv ? 2 + v : var;
                 near_sum<K, F32>(B.n, derive, rv, mk, nwords, 1.0 / sv, colx, sh);   // (sv is a power of two)
                 // of a tile of both sets only set v's columns, over their own intervals
