@@ -655,7 +655,7 @@ struct WaveStage64 {
 // An interval of the tile's columns in f, of one range (kFarRanges); hi < lo: no columns
 struct NearInterval {
     double c, r;          // centre, half width
-    float lo, hi, thr;    // thr: the least |z - lo| + |z - hi| of a pole outside the ellipse
+    float lo, hi, thr;    // thr: the least |z - lo| + |z - hi| of a pole outside the ellipse (NaN: none is)
 };
 
 template <int K, bool F32>
@@ -974,6 +974,7 @@ __device__ double tree_to_column(NearShared<K, F32> &sh, int rv, double f) {
         for (int w = 0; w < kThreads / 64; ++w) out += sh.column[w][tid];
         for (int i = Tree::leaves + leaf; i >= 1; i >>= 1) {
             const NearInterval &I = sh.iv[rv][i];
+            if (!(I.thr >= 0.0f)) continue;   // no nodes taken (c and r may not be finite)
             const double u = I.r > 0.0 ? (f - I.c) / I.r : 0.0, u2 = 2.0 * u;
             double b1 = 0.0, b2 = 0.0;   // Clenshaw
 #pragma unroll
@@ -1060,11 +1061,12 @@ __global__ __launch_bounds__(kThreads, 4) void alpha_near_kernel(AlphaArgs args)
         I.hi = static_cast<float>(hi);
         I.c = 0.5 * (lo + hi);
         I.r = 0.5 * (hi - lo);
-        // The margin covers the FP32 roundings of lo, hi and the poles; f < 0: never outside.  A
+        // The margin covers the FP32 roundings of lo, hi and the poles.  No nodes (thr NaN: no pole is
+        // outside) where f < 0, or past where the FP32 distances' squares overflow (f infinite).  A
         // node's f is rounded to 2^-53 c, which moves a term by up to about 2^-53 c / r of itself:
         // FP64 mode takes no nodes in narrow intervals.
-        const bool use = lo >= 0.0 && (F32 || 64.0 * I.r >= I.c);
-        I.thr = use ? static_cast<float>(I.r * (node_rho<F32>() + 1.0 / node_rho<F32>()) + 1.0e-6 * hi) : INFINITY;
+        const bool use = lo >= 0.0 && hi < 1.0e15 && (F32 || 64.0 * I.r >= I.c);
+        I.thr = use ? static_cast<float>(I.r * (node_rho<F32>() + 1.0 / node_rho<F32>()) + 1.0e-6 * hi) : NAN;
     }
     for (int e = tid; e < kFarMom; e += kThreads) {
         double s = 0.0;
