@@ -193,10 +193,12 @@ def _check_orton_freqs(catalog, freqs):
 
 
 def nh3_order(freqs):
-    """Column order of nh3_hs's output: request indices <= 30 GHz, then > 30 GHz."""
+    """Column order of nh3_hs's output: request indices <= 30 GHz, then the others (NaN among them:
+    every column has a place, the kernels read one entry for each)."""
     f = np.asarray(freqs, dtype=np.float64)
-    lo = np.where(f <= F_SPLIT)[0]
-    hi = np.where(f > F_SPLIT)[0]
+    low = f <= F_SPLIT
+    lo = np.where(low)[0]
+    hi = np.where(~low)[0]
     return np.concatenate([lo, hi]), len(lo)
 
 
