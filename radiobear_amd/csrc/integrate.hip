@@ -424,13 +424,16 @@ __global__ __launch_bounds__(kWaves * kLanes) void integrate_f32_kernel(IntArgs 
 // exactly.  The two sums are taken by path point,
 // sum_i (W_i + W_{i+1}) h_i = sum_p W_p (h_{p-1} + h_p) (W_0 = 0, h_n = 0), so a run needs
 // nothing of its neighbours but the starting tau.  All FP64, also where the table is FP32.  The
-// tau cut ends each thread's walk at the first point past it.
+// tau cut ends a thread's walk at the first point past it, and the runs after the first one it ends
+// add nothing: their starting tau is summed over what lies past the cut, and absorption below 0 or
+// NaN there would bring it back.
 constexpr int kSegThreads = 1024;
 template <class AT, int MODE, int COLS>
 __global__ __launch_bounds__(kSegThreads) void integrate_segments_kernel(IntArgs A, int colgroups) {
     constexpr int SEGS = kSegThreads / COLS, W = kSegThreads / kLanes;
     __shared__ double etab[kExpTab];
     __shared__ double part[2][W][COLS];
+    __shared__ int halt[W][COLS];   // a run of the wavefront passed the cut
     const int col = threadIdx.x % COLS, seg = threadIdx.x / COLS;
     const int wave = threadIdx.x / kLanes, lane = threadIdx.x % kLanes;
     if (MODE == 0 && threadIdx.x < kExpTab) etab[threadIdx.x] = kExp2Tab[threadIdx.x];
@@ -477,8 +480,10 @@ __global__ __launch_bounds__(kSegThreads) void integrate_segments_kernel(IntArgs
     if (lane >= COLS) tau += own;
     const double cut = (A.tau_cut > 0.0 && !bad) ? A.tau_cut : 0.0;
     double intW = 0.0, num = 0.0, a0 = before;
+    bool past = false;
     for (int p = p0; p < p1; ++p) {
-        if (cut > 0.0 && tau > cut) break;
+        past = cut > 0.0 && tau > cut;
+        if (past) break;
         const double a1 = static_cast<double>(al[p * nf]);
         const double hb = h[p - 1];
         tau = tau + (a0 + a1) * hb;
@@ -489,14 +494,20 @@ __global__ __launch_bounds__(kSegThreads) void integrate_segments_kernel(IntArgs
         a0 = a1;
     }
 #pragma unroll
-    for (int o = COLS; o < kLanes; o <<= 1) {
-        intW += __shfl_xor(intW, o, kLanes);
-        num += __shfl_xor(num, o, kLanes);
+    for (int o = COLS; o < kLanes; o <<= 1) {   // (earlier runs in the lanes without bit o)
+        const bool later = lane & o;
+        const double oW = __shfl_xor(intW, o, kLanes), onum = __shfl_xor(num, o, kLanes);
+        const bool opast = __shfl_xor(static_cast<int>(past), o, kLanes);
+        const bool stop = later ? opast : past;
+        intW = stop ? (later ? oW : intW) : intW + oW;
+        num = stop ? (later ? onum : num) : num + onum;
+        past = past || opast;
     }
     __syncthreads();   // part[0] has been read
     if (lane < COLS) {
         part[0][wave][col] = intW;
         part[1][wave][col] = num;
+        halt[wave][col] = past;
     }
     __syncthreads();
     if (threadIdx.x >= COLS || !ok) return;
@@ -504,6 +515,7 @@ __global__ __launch_bounds__(kSegThreads) void integrate_segments_kernel(IntArgs
     for (int w = 0; w < W; ++w) {
         intW += part[0][w][col];
         num += part[1][w][col];
+        if (halt[w][col]) break;
     }
     const size_t o = static_cast<size_t>(ray) * A.nf + (A.cols ? A.cols[j] : j);
     double Tb;
