@@ -348,6 +348,7 @@ __global__ __launch_bounds__(kRayThreads) void raypath_kernel(RayArgs A) {
     const double z1 = start + -0.005;
     const double dz = z1 - start;
     const double flat = 1.0 - G.ratio * G.ratio;
+    const bool shell = rNorm != 0.0 && fabs(rNorm) < INFINITY;   // (else no trial is below it)
     auto trial = [&](int i) { return (i == 0) ? start : ((i == 1) ? z1 : start + i * dz); };
     int hit = -1;
     for (int i0 = 0; i0 < ntrial && hit < 0; i0 += L) {   // L trials at a time, the first below taken
@@ -355,7 +356,7 @@ __global__ __launch_bounds__(kRayThreads) void raypath_kernel(RayArgs A) {
         const V3 bv = mat(G.M, V3{b0, b1, trial(i)});
         const double q = dot(bv, bv), Y = bv.y * bv.y;
         // q < f^2 times q > 0 (1e-6 rad at y == 0)
-        const bool below = i < ntrial && q * q < fma(-flat, bv.y == 0.0 ? kLat0 * q : Y, q);
+        const bool below = shell && i < ntrial && q * q < fma(-flat, bv.y == 0.0 ? kLat0 * q : Y, q);
         if constexpr (L == 1) {
             if (below) hit = i;
         } else {
