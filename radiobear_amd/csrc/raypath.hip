@@ -250,7 +250,7 @@ __device__ inline int parallel_steps(const RayArgs &A, const double *Rl, int nl,
                     const double dR = (win[i] - win[i + 1]) * (win[i] + win[i + 1]);
                     const double v = f2 * dR, un = u - v, Sn = sqrt_km2(d1sq + un);
                     const double ds = v * rcp_pos(S + Sn);
-                    if (neg == n && ds < 0.0) neg = k;
+                    if (neg == n && v < 0.0 && S >= 0.0) neg = k;   // ds < 0, also where un is infinite
                     stage[c][i] = ds * unit;
                     // 1 - d f^2/du dR (a derivative: the estimate of 1 / S will do)
                     D *= fma(-flat * dR * iq, fma(ys, __builtin_amdgcn_rcp(S), y * y * iq), 1.0);
