@@ -43,13 +43,16 @@ def as_device(x, dtype=torch.float64):
     return t.contiguous()
 
 
+_PACKED = (np.float64, np.float32, np.int64, np.int32)
+
+
 def as_device_all(*xs):
     """as_device of each; host arrays cross in one copy (a copy from pageable memory costs about
     20 us whatever its size), each then starting at a multiple of 512 bytes as tensors do."""
     host = [i for i, x in enumerate(xs) if not isinstance(x, torch.Tensor)]
-    if len(host) < 2:
+    arrays = [np.asarray(xs[i]) for i in host]
+    if len(host) < 2 or any(a.dtype not in _PACKED for a in arrays):   # (as_device refuses what it refuses)
         return [as_device(x) for x in xs]
-    arrays = [np.asarray(xs[i], dtype=np.float64) for i in host]
     at = np.concatenate([[0], np.cumsum([-(-a.size // 64) * 64 for a in arrays])])
     packed = np.zeros(int(at[-1]))
     for k, a in zip(at, arrays):
@@ -363,6 +366,8 @@ def _rays(b):
 
 def raypaths(planet, R, N, b, units='half_cm'):
     """Ray paths for impact parameters b (nray, 2): (ds (nray, nl-1) float64, nsteps (nray,) int32)."""
+    if not isinstance(b, torch.Tensor):
+        b = np.asarray(b, dtype=np.float64).reshape(-1, 2)
     R, N, b = as_device_all(R, N, b)
     b = _rays(b)
     nl = R.shape[0]
