@@ -638,8 +638,9 @@ def main():
         roof = {'kernel': dom, 'bound': 'valu', 'achieved': achieved, 'peak': PEAK['fp32'], 'unit': 'TFLOP/s',
                 'frac': achieved / PEAK['fp32'], 'traffic': None,
                 'algorithmic_flop_per_launch': flop,
-                'basis': 'FLOP of the direct sum over every (line, layer, frequency); the far-line series path '
-                         'sums about a third of those pairs and adds the rest as per-tile power series'}
+                'basis': 'FLOP of the direct sum over every (line, layer, frequency), most of which the far-line '
+                         'series path does not execute: it adds far lines as per-tile power series and sums '
+                         'near ones at the nodes of column intervals'}
     else:
         steps = float(np.sum(np.maximum(ns - 1, 0)))
         flop = steps * prob.nf * FLOP_RT_STEP

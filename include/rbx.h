@@ -293,7 +293,8 @@ int rbx_alpha_tangent_workspace_size(const rbx_catalog *cat, const rbx_absorbers
  * b               [nray][2] impact parameters (fraction of R[0])
  * ds              [nray][ld] step lengths; out_units 0: km (Ray.ds),
  *                 1: half step in cm ((ds*1e3/1e-2)/2, what rbx_integrate consumes)
- * nsteps          [nray] entries of ds used; -1 = off planet (Ray.ds None)
+ * nsteps          [nray] entries of ds used; -1 = off planet (Ray.ds None).  What a row holds
+ *                 past them is unspecified (entries up to nl - 1 may be written)
  * ld >= nl - 1.
  */
 int rbx_raypaths(const rbx_planet *planet, const double *R, const double *N, int nl,
@@ -306,7 +307,9 @@ int rbx_raypaths(const rbx_planet *planet, const double *R, const double *N, int
  * hds, ld, nsteps from rbx_raypaths with out_units 1
  * mode            0: point ray, W = alpha e^-tau; 1: disc average, W = 2 alpha E2(tau)
  * precision       RBX_FP64 or RBX_FP32 (how e^-tau is evaluated; tau is FP64 in both)
- * tau_cut         stop a ray's frequency group once every tau > tau_cut (<= 0: never)
+ * tau_cut         stop a ray's frequency group once every tau > tau_cut (<= 0: never; requests of
+ *                 few rays stop each frequency by itself, at the first step past it).  A ray
+ *                 whose path holds a NaN half step or temperature is never cut
  * Tb              [nray][nf] K; intW [nray][nf] integrated weight or NULL
  */
 int rbx_integrate(const void *alpha, int alpha_precision, const double *T, int nl, int nf,

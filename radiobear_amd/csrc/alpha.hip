@@ -1752,9 +1752,12 @@ static int alpha_split(const AlphaArgs &A, const rbx_launch &L, int K, int preci
 // kSeriesMaxWorkspace for requests of at least kSeriesMinTiles tiles of the direct sums' width, and of
 // fewer where the direct sums are long enough that the two passes' launches (about 50 us) pay.  (One
 // 20-frequency tile of 150 layers took 0.37 ms per step with the series against 0.21 ms without.)
-// Direct -> series, 10000 lines unless said: FP64 300 layers x 130 columns 419 -> 430 us, x 200
-// 528 -> 432, x 256 581 -> 450, 100 x 130 x 800 lines 53 -> 110 us; FP32 300 x 256 305 -> 381, 300 x 400
-// 425 -> 386 (7 tiles), 800 x 300 x 20000 lines 1522 -> 968.
+// Direct -> series, 10000 lines unless said: FP64 300 layers x 130 columns 419 -> 430 us, x 256 581 ->
+// 450, 100 x 130 x 800 lines 53 -> 110 us; FP32 300 x 256 305 -> 381, 800 x 300 x 20000 lines 1522 -> 968;
+// of four tiles FP64 300 x 200 528 -> 432, FP32 300 x 400 425 -> 386 (from there on the work is not
+// looked at, and short lists or few layers lose what 100 x 130 x 800 does).  Against 64 bits the FP64
+// series' error in those requests is half to nine tenths of the direct sums' in the mean square (their
+// roundings grow with the lines they add), its largest entry up to 5e-14 against 2e-14.
 constexpr size_t kSeriesMaxWorkspace = size_t(4) << 30;
 constexpr int kSeriesMinTiles = 4;
 static bool series_on(const AlphaArgs &A, const rbx_launch &L, int precision) {

@@ -2,8 +2,8 @@
 
 Mirrors radiobear/raypath.py:20-273: ``compute_ds`` returns a ``Ray`` with the
 step lengths ``ds`` (km) and the layer of each step, or ``ds = None`` when the
-ray misses the planet.  The stepping runs in rbx_raypaths (one GPU thread per
-ray); ``batch`` traces many rays in one launch and keeps the result on the
+ray misses the planet.  The stepping runs in rbx_raypaths (a ray's steps
+split over 32 lanes, or a GPU thread per ray for many rays); ``batch`` traces many rays in one launch and keeps the result on the
 device for the integration kernel.
 """
 import numpy as np
