@@ -306,7 +306,8 @@ int rbx_raypaths(const rbx_planet *planet, const double *R, const double *N, int
  * T               [nl] K
  * hds, ld, nsteps from rbx_raypaths with out_units 1
  * mode            0: point ray, W = alpha e^-tau; 1: disc average, W = 2 alpha E2(tau)
- * precision       RBX_FP64 or RBX_FP32 (how e^-tau is evaluated; tau is FP64 in both)
+ * precision       RBX_FP64 or RBX_FP32 (how e^-tau is evaluated; tau is FP64 in both, and
+ *                 requests of few rays take FP64 weights in either)
  * tau_cut         stop a ray's frequency group once every tau > tau_cut (<= 0: never; requests of
  *                 few rays stop each frequency by itself, at the first step past it).  A ray
  *                 whose path holds a NaN half step or temperature is never cut
